@@ -280,45 +280,51 @@ int launch_argmax(cw_ctx *ctx, const float *logits, int n, uint32_t *out_dev, vo
 
 // ---- batched prefill (M positions per launch)
 
-// y[M][N] = x[M][K] . W[N][K]^T with x given as bf16 hi/lo rows and W split
-// GGUF Q4_0; EPI_SWIGLU reads a second matrix (B) and stores silu(A x) * (B x).
+// y[M][N] = x[M][K] . W[N][K]^T with x given as its split image (q4_gemm.hip)
+// and W split GGUF Q4_0; EPI_SWIGLU reads a second matrix (B) and stores
+// silu(A x) * (B x).
 struct GemmArgs {
-    const uint16_t *xhi, *xlo;  // [M][K] f16 bits, row m scaled by 1 / rowscale[m]
-                                // (allocated for gemm_x_elems(M, K))
+    const uint16_t *img;        // x image, gemm_img_elems(M, K) elements
     const float *rowscale;      // [M] powers of two
     const uint16_t *sA;
     const uint8_t *qA;
     const uint16_t *sB;
     const uint8_t *qB;
+    int s_stride;               // set by launch_q4_gemm: blocks per row of sA / sB
+    uint16_t *s_pad;            // room for padded scales (gemm_spad_elems), else null
     const float *resid;  // EPI_ADD: [M][N]
     float *y;            // [M][N]
     int M, N, K;
     float *part;         // split-K partials (null: no split)
     size_t part_floats;  // capacity of part
-    // optional: y also split for the next GEMM, exactly as launch_split_rows
-    // (x = y, norm_w = next_norm) would; with split K it is done by the
-    // reduction of the partials, in the same pass
-    bool split_next;
-    const float *next_norm;
-    float next_eps;
-    uint16_t *next_hi, *next_lo;
-    float *next_rowscale;
 };
-// K splits the GEMM uses for this shape (the partial workspace holds
-// splits * M * N floats)
-int gemm_splits(const cw_ctx *ctx, Epi epi, int M, int N, int K);
-// Elements each of GemmArgs::xhi / xlo must hold for M rows of K: whole
-// 128-row tiles plus one block (the GEMM's DMA reads them; rows past M are
-// never stored to y, so they need no values)
-size_t gemm_x_elems(int M, int K);
+// Elements of the split image of M rows of K (rows are padded to whole row
+// tiles: the GEMM's DMA reads them; rows past M are never stored to y, so
+// they need no values)
+size_t gemm_img_elems(int M, int K);
+// padded scales of N rows of K, for matrices whose scales the GEMM cannot
+// read in pairs (0: not needed)
+size_t gemm_spad_elems(int N, int K, const void *scales);
+// floats of split-K partials the GEMM's plan takes for this shape (0: none);
+// with less room it takes the best plan that fits
+size_t gemm_part_floats(const cw_ctx *ctx, Epi epi, int M, int N, int K);
 // token ids on the device (validated < vocab by the caller)
 int launch_embed_rows(cw_ctx *ctx, const float *table, int dim, const uint32_t *tok_dev, int n,
                       float *out);
+// The split image of rows of x, RMS-normalised with norm_w when set.
 int launch_split_rows(cw_ctx *ctx, const float *x, const float *norm_w, float eps, int rows, int K,
-                      uint16_t *hi, uint16_t *lo, float *rowscale);
-// kept_splits (optional): with split K, leave the partials in a.part
-// unreduced and set *kept_splits = K splits (0 when y was written)
-int launch_q4_gemm(cw_ctx *ctx, Epi epi, const GemmArgs &a, int *kept_splits = nullptr);
+                      uint16_t *img, float *rowscale);
+// *splits = 0 when y was written, else the K splits whose partials are in
+// a.part (a.resid not yet added): [split][M][N], for SwiGLU [split][gate |
+// up][M][N].
+int launch_q4_gemm(cw_ctx *ctx, Epi epi, GemmArgs a, int *splits);
+// y = [resid +] the sum in order of a.part's `splits` partials
+int launch_gemm_reduce(cw_ctx *ctx, const GemmArgs &a, int splits);
+// The GEMM's result (its partials summed in the same pass) as the next GEMM's
+// split image, RMS-normalised with norm_w when set; y holds it too, but for
+// SwiGLU partials.
+int launch_reduce_split(cw_ctx *ctx, Epi epi, const GemmArgs &a, int splits, const float *norm_w,
+                        float eps, uint16_t *img, float *rowscale);
 // qkv: [M][q | k | v] rows, or (splits > 0) the sum in order of `splits`
 // partials part[s][M][q | k | v] (gemm_reduce_kernel's sum)
 int launch_qk_rope_kv(cw_ctx *ctx, const float *qkv, const float *qn, const float *kn, float eps,

@@ -92,8 +92,9 @@ struct cw_model {
     int pf_cap = 0;
     float *pf_hidden = nullptr, *pf_qkv = nullptr, *pf_q = nullptr, *pf_attn = nullptr,
           *pf_act = nullptr;
-    uint16_t *pf_hi = nullptr, *pf_lo = nullptr;
-    float *pf_rowscale = nullptr;  // per-row powers of two of the GEMM operand split
+    uint16_t *pf_img = nullptr;    // the current GEMM operand's split image
+    float *pf_rowscale = nullptr;  // its per-row powers of two
+    uint16_t *pf_spad = nullptr;   // padded scales (matrices that need them)
     float *pf_part = nullptr;  // split-K partials of the prefill GEMMs
     size_t pf_part_floats = 0;
     std::vector<void *> pf_allocs;
@@ -491,6 +492,9 @@ int ensure_prefill(cw_model *m, int n) {
     for (void *p : m->pf_allocs) CW_HIP(hipFree(p));
     m->pf_allocs.clear();
     m->pf_cap = 0;
+    m->pf_part = nullptr;
+    m->pf_part_floats = 0;
+    m->pf_spad = nullptr;
     const auto &c = m->cfg;
     const size_t wide = std::max({(size_t)c.dim, (size_t)m->q_dim, (size_t)c.hidden});
     auto al = [&](size_t bytes, void **out) -> int {
@@ -503,47 +507,41 @@ int ensure_prefill(cw_model *m, int n) {
     CW_TRY(al((size_t)n * m->q_dim * 4, (void **)&m->pf_q));
     CW_TRY(al((size_t)n * m->q_dim * 4, (void **)&m->pf_attn));
     CW_TRY(al((size_t)n * c.hidden * 4, (void **)&m->pf_act));
-    CW_TRY(al(gemm_x_elems(n, (int)wide) * 2, (void **)&m->pf_hi));
-    CW_TRY(al(gemm_x_elems(n, (int)wide) * 2, (void **)&m->pf_lo));
+    CW_TRY(al(gemm_img_elems(n, (int)wide) * 2, (void **)&m->pf_img));
     CW_TRY(al((size_t)n * 4, (void **)&m->pf_rowscale));
-    // split-K workspace: the largest splits x M x N of the unfused GEMMs
-    size_t part = 0;
-    const int qkv_n = m->q_dim + 2 * m->kv_dim;
-    const int shapes[3][2] = {{qkv_n, c.dim}, {c.dim, m->q_dim}, {c.dim, c.hidden}};  // N, K
-    for (const auto &sh : shapes) {
-        const int S = gemm_splits(m->ctx, EPI_ADD, n, sh[0], sh[1]);
-        if (S > 1) part = std::max(part, (size_t)S * n * sh[0]);
+    // split-K partials of the largest plan (for n and for shorter prompts,
+    // whose plans split further), and room for padded scales
+    struct Shape {
+        Epi epi;
+        int N, K;
+        const uint16_t *s;
+    };
+    const Layer &L = m->layers[0];
+    const Shape shapes[] = {{EPI_STORE, m->q_dim + 2 * m->kv_dim, c.dim, L.qkv.s},
+                            {EPI_ADD, c.dim, m->q_dim, L.wo.s},
+                            {EPI_SWIGLU, c.hidden, c.dim, L.gate.s},
+                            {EPI_ADD, c.dim, c.hidden, L.down.s}};
+    size_t part = 0, spad = 0;
+    for (const Shape &s : shapes) {
+        for (int k = n; k > 0; k /= 2)
+            part = std::max(part, gemm_part_floats(m->ctx, s.epi, k, s.N, s.K));
+        const int mats = s.epi == EPI_SWIGLU ? 2 : 1;
+        spad = std::max(spad, mats * gemm_spad_elems(s.N, s.K, s.s));
     }
-    if (part > 0) {
-        CW_TRY(al(part * 4, (void **)&m->pf_part));
-        m->pf_part_floats = part;
-    }
+    if (part > 0) CW_TRY(al(part * 4, (void **)&m->pf_part));
+    if (spad > 0) CW_TRY(al(spad * 2, (void **)&m->pf_spad));
+    m->pf_part_floats = part;
     m->pf_cap = n;
     return CW_OK;
 }
 
-// One linear layer of the batched forward: rows of x (optionally
-// RMS-normalised) through a Q4_0 matrix pair or single matrix.
-// y[n][out] = [resid +] (RMSNorm?) x . W^T on the batched GEMM.  x_split:
-// pf_hi / pf_lo / pf_rowscale already hold x's split (the previous GEMM left
-// it); next_split: leave y's split there for the next GEMM, RMS-normalised
-// with next_norm when set.
-int pf_linear(cw_model *m, const float *x, const float *norm_w, int n, int K, Epi epi,
-              const Q4W &w, const Q4W *w2, const float *resid, float *y, bool x_split = false,
-              bool next_split = false, const float *next_norm = nullptr,
-              int *kept_splits = nullptr) {
-    if (!x_split)
-        CW_TRY(launch_split_rows(m->ctx, x, norm_w, m->cfg.eps, n, K, m->pf_hi, m->pf_lo,
-                                 m->pf_rowscale));
+// The batched GEMM of one linear layer: y[n][out] = [resid +] x . W^T (SwiGLU
+// of two matrices), x being the split image in pf_img.  *splits as
+// launch_q4_gemm leaves it; the arguments come back for the pass that follows.
+int pf_gemm(cw_model *m, int n, int K, Epi epi, const Q4W &w, const Q4W *w2, const float *resid,
+            float *y, GemmArgs *out, int *splits) {
     GemmArgs a{};
-    a.split_next = next_split;
-    a.next_norm = next_norm;
-    a.next_eps = m->cfg.eps;
-    a.next_hi = m->pf_hi;
-    a.next_lo = m->pf_lo;
-    a.next_rowscale = m->pf_rowscale;
-    a.xhi = m->pf_hi;
-    a.xlo = m->pf_lo;
+    a.img = m->pf_img;
     a.rowscale = m->pf_rowscale;
     a.sA = w.s;
     a.qA = w.q;
@@ -551,6 +549,7 @@ int pf_linear(cw_model *m, const float *x, const float *norm_w, int n, int K, Ep
         a.sB = w2->s;
         a.qB = w2->q;
     }
+    a.s_pad = m->pf_spad;
     a.resid = resid;
     a.y = y;
     a.M = n;
@@ -558,7 +557,8 @@ int pf_linear(cw_model *m, const float *x, const float *norm_w, int n, int K, Ep
     a.K = K;
     a.part = m->pf_part;
     a.part_floats = m->pf_part_floats;
-    return launch_q4_gemm(m->ctx, epi, a, kept_splits);
+    *out = a;
+    return launch_q4_gemm(m->ctx, epi, a, splits);
 }
 
 // With taps on: row `row` of a batched [n][floats] buffer into a tap.
@@ -576,30 +576,41 @@ int enqueue_prefill(cw_model *m, int n, int start) {
     cw_ctx *ctx = m->ctx;
     const auto &c = m->cfg;
     CW_TRY(launch_embed_rows(ctx, m->embed, c.dim, m->prompt_dev, n, m->pf_hidden));
+    const float eps = c.eps;
+    // a GEMM's result as the next one's operand, in one pass
+    auto to_image = [&](Epi epi, const GemmArgs &a, int splits, const float *norm_w) {
+        return launch_reduce_split(ctx, epi, a, splits, norm_w, eps, m->pf_img, m->pf_rowscale);
+    };
+    GemmArgs g{};
+    int splits = 0;
+    CW_TRY(launch_split_rows(ctx, m->pf_hidden, m->layers[0].attn_norm, eps, n, c.dim, m->pf_img,
+                             m->pf_rowscale));
     for (int i = 0; i < c.n_layers; ++i) {
         Layer &L = m->layers[i];
         void *kc = (char *)m->kcache + (size_t)i * m->kv_layer_bytes;
         void *vc = (char *)m->vcache + (size_t)i * m->kv_layer_bytes;
-        // the split of the layer's input: the previous layer's down GEMM left
-        // it; with split K the partials go straight to the QK-norm + RoPE pass
-        int qkv_splits = 0;
-        CW_TRY(pf_linear(m, m->pf_hidden, L.attn_norm, n, c.dim, EPI_STORE, L.qkv, nullptr,
-                         nullptr, m->pf_qkv, i > 0, false, nullptr, &qkv_splits));
-        CW_TRY(launch_qk_rope_kv(ctx, m->pf_qkv, L.q_norm, L.k_norm, c.eps, m->cos_t, m->sin_t, n,
+        // (with split K the partials go straight to the QK-norm + RoPE pass)
+        CW_TRY(pf_gemm(m, n, c.dim, EPI_STORE, L.qkv, nullptr, nullptr, m->pf_qkv, &g, &splits));
+        CW_TRY(launch_qk_rope_kv(ctx, m->pf_qkv, L.q_norm, L.k_norm, eps, m->cos_t, m->sin_t, n,
                                  c.n_heads, c.n_kv_heads, start, c.kv_dtype, m->pf_q, kc, vc,
-                                 qkv_splits ? m->pf_part : nullptr, qkv_splits));
+                                 splits ? m->pf_part : nullptr, splits));
         CW_TRY(tap_row(m, m->tap_q + (size_t)i * m->q_dim, m->pf_q, n - 1, m->q_dim));
         CW_TRY(launch_attn_prefill(ctx, m->pf_q, kc, vc, n, c.n_heads, c.n_kv_heads, start,
                                    m->pf_attn));
-        CW_TRY(pf_linear(m, m->pf_attn, nullptr, n, m->q_dim, EPI_ADD, L.wo, nullptr,
-                         m->pf_hidden, m->pf_hidden, false, true, L.ffn_norm));
+        CW_TRY(launch_split_rows(ctx, m->pf_attn, nullptr, eps, n, m->q_dim, m->pf_img,
+                                 m->pf_rowscale));
+        CW_TRY(pf_gemm(m, n, m->q_dim, EPI_ADD, L.wo, nullptr, m->pf_hidden, m->pf_hidden, &g,
+                       &splits));
+        CW_TRY(to_image(EPI_ADD, g, splits, L.ffn_norm));
         CW_TRY(tap_row(m, m->tap_post + (size_t)i * c.dim, m->pf_hidden, n - 1, c.dim));
-        CW_TRY(pf_linear(m, m->pf_hidden, L.ffn_norm, n, c.dim, EPI_SWIGLU, L.gate, &L.up,
-                         nullptr, m->pf_act, true));
-        const bool more = i + 1 < c.n_layers;
-        CW_TRY(pf_linear(m, m->pf_act, nullptr, n, c.hidden, EPI_ADD, L.down, nullptr,
-                         m->pf_hidden, m->pf_hidden, false, more,
-                         more ? m->layers[i + 1].attn_norm : nullptr));
+        CW_TRY(pf_gemm(m, n, c.dim, EPI_SWIGLU, L.gate, &L.up, nullptr, m->pf_act, &g, &splits));
+        CW_TRY(to_image(EPI_SWIGLU, g, splits, nullptr));
+        CW_TRY(pf_gemm(m, n, c.hidden, EPI_ADD, L.down, nullptr, m->pf_hidden, m->pf_hidden, &g,
+                       &splits));
+        if (i + 1 < c.n_layers)
+            CW_TRY(to_image(EPI_ADD, g, splits, m->layers[i + 1].attn_norm));
+        else if (splits)
+            CW_TRY(launch_gemm_reduce(ctx, g, splits));
         CW_TRY(tap_row(m, m->tap_out + (size_t)i * c.dim, m->pf_hidden, n - 1, c.dim));
     }
     return CW_OK;

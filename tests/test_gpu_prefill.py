@@ -47,6 +47,41 @@ def test_q4_gemm_vs_oracle(ctx, m, in_f, out_f):
     assert worst <= 1e-4, worst
 
 
+# Edges of the GEMM's tiles (16, 32 and 64 rows; 64, 128 and 256 columns), of
+# its scale groups (8 blocks) and K splits, one row and one column included
+GEMM_EDGES = [(m, k, n) for m in (1, 15, 17, 33, 63, 65, 129)
+              for k, n in ((32, 1), (288, 63), (2048, 129))] + \
+             [(2, 12288, 65), (16, 40960, 64), (31, 4128, 257), (260, 1024, 300)]
+
+
+@pytest.mark.parametrize("m,in_f,out_f", GEMM_EDGES)
+def test_q4_gemm_tile_edges(ctx, m, in_f, out_f):
+    """Every element against an f64 product of the exactly dequantized
+    weights.  The operands are exact to 2^-23 and the sums are f32: the same
+    bound as above, 2e-5 * sum_k |w x| (2^-24 per add over at most 1,280
+    blocks stays below it by a factor of 4)."""
+    s, q = cw.synth_q4(cw.synth_key(25, f"e{out_f}x{in_f}"), out_f, in_f, 0.02)
+    x = cw.synth_normal_f32(cw.synth_key(25, f"ex{m}x{in_f}"), m * in_f).reshape(m, in_f)
+    y = ctx.q4_gemm(ctx.storage(x), m, ctx.storage(s), ctx.storage(q), in_f, out_f).download()
+    w = orc.dequant_q4_0_soa(s, q).reshape(out_f, in_f).astype(np.float64)
+    x64 = x.astype(np.float64)
+    err = np.abs(y.reshape(m, out_f) - x64 @ w.T)
+    assert np.all(err <= 2e-5 * (np.abs(x64) @ np.abs(w).T) + 1e-30)
+
+
+def test_q4_gemm_scales_at_odd_addresses(ctx):
+    """Scales at an address that is a multiple of 2 only give the same bits as
+    aligned ones (they are copied to aligned rows first)."""
+    m, in_f, out_f = 20, 512, 96
+    s, q = cw.synth_q4(cw.synth_key(26, "w"), out_f, in_f, 0.02)
+    x = ctx.storage(cw.synth_normal_f32(cw.synth_key(26, "x"), m * in_f))
+    qd = ctx.storage(q)
+    ref = ctx.q4_gemm(x, m, ctx.storage(s), qd, in_f, out_f).download()
+    moved = ctx.storage(np.concatenate([np.zeros(1, np.uint16), s.reshape(-1)]))
+    at2 = cw.DeviceArray(ctx, s.shape, np.uint16, moved.ptr + 2)
+    assert np.array_equal(ref, ctx.q4_gemm(x, m, at2, qd, in_f, out_f).download())
+
+
 # the four projection shapes of one 8B layer at the 512-token workload:
 # QKV (4096 -> 6144), O (4096 -> 4096), gate/up (4096 -> 12288, each) and
 # down (12288 -> 4096); (m, in_f, out_f).  These run the split-K and tile
@@ -178,6 +213,46 @@ def test_prefill_small_model(ctx, P):
     assert np.array_equal(toks, ref[1:N + 1]), (toks, ref[1:N + 1])
     m.close()
     o.close()
+
+
+@pytest.mark.parametrize("P", [2, 20, 40, 70])
+def test_prefill_odd_widths(ctx, P):
+    """Widths that are not whole scale groups (288 and 544: 9 and 17 blocks)
+    through every projection, for prompts on either side of the 16, 32 and 64
+    row tiles: logits within 1e-3 of the oracle's per-token forward."""
+    cfg = small_f16(P + 2, dim=288, hidden=544)
+    weights = cw.synthetic_weights(cfg, 82)
+    prompt = cw.synth_tokens(cw.synth_key(82, f"p{P}"), P, cfg.vocab)
+    m = cw.Model(ctx, cfg)
+    m.set_weights(weights)
+    m.finalize()
+    o = orc.OracleModel(cfg, weights)
+    nxt = m.prefill(prompt)
+    ref_logits = oracle_prompt_logits(o, prompt)
+    diff = float(np.max(np.abs(m.logits() - ref_logits)))
+    assert diff <= LOGIT_TOL, diff
+    assert nxt == int(np.argmax(ref_logits))
+    m.close()
+    o.close()
+
+
+def test_prefill_after_a_longer_one(ctx):
+    """A shorter prompt through the buffers of a longer one (its plans split K
+    further) gives the logits of a fresh model's."""
+    cfg = small_f16(300)
+    weights = cw.synthetic_weights(cfg, 83)
+    prompt = cw.synth_tokens(cw.synth_key(83, "p"), 280, cfg.vocab)
+    logits = []
+    for first in (280, 0):
+        m = cw.Model(ctx, cfg)
+        m.set_weights(weights)
+        m.finalize()
+        if first:
+            m.prefill(prompt)
+        m.prefill(prompt[:150])
+        logits.append(m.logits())
+        m.close()
+    assert float(np.max(np.abs(logits[0] - logits[1]))) <= 1e-4
 
 
 @pytest.mark.parametrize("n_heads,n_kv", [(4, 4), (8, 1), (16, 2)])
