@@ -153,6 +153,33 @@ struct same_type {
     using type = T;
 };
 
+__device__ __forceinline__ float add(float a, float b) { return a + b; }
+__device__ __forceinline__ float4 add(float4 a, float4 b) {
+    return make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w);
+}
+
+// The sum in order of the S >= 1 partials at p, p + stride, ...: four
+// requested at a time, so that no load waits for another's sum.
+template <typename T>
+__device__ __forceinline__ T sum_parts(const float *p, int S, size_t stride) {
+    auto at = [&](int s) { return *reinterpret_cast<const T *>(p + (size_t)s * stride); };
+    T v = at(0);
+    int s = 1;
+    for (; s + 4 <= S; s += 4) {
+        const T a = at(s), b = at(s + 1), c = at(s + 2), d = at(s + 3);
+        v = add(add(add(add(v, a), b), c), d);
+    }
+    if (s + 3 == S) {
+        const T a = at(s), b = at(s + 1), c = at(s + 2);
+        return add(add(add(v, a), b), c);
+    }
+    if (s + 2 == S) {
+        const T a = at(s), b = at(s + 1);
+        return add(add(v, a), b);
+    }
+    return s < S ? add(v, at(s)) : v;
+}
+
 // Enqueue fn on ctx->stream.  While profiling, the dispatch itself stamps a
 // pair of events at the kernel's start and end (hipExtLaunchKernel), so the
 // profile holds kernel execution time, as a kernel trace does, with no
@@ -308,12 +335,14 @@ size_t gemm_spad_elems(int N, int K, const void *scales);
 // floats of split-K partials the GEMM's plan takes for this shape (0: none);
 // with less room it takes the best plan that fits
 size_t gemm_part_floats(const cw_ctx *ctx, Epi epi, int M, int N, int K);
-// token ids on the device (validated < vocab by the caller)
-int launch_embed_rows(cw_ctx *ctx, const float *table, int dim, const uint32_t *tok_dev, int n,
-                      float *out);
 // The split image of rows of x, RMS-normalised with norm_w when set.
 int launch_split_rows(cw_ctx *ctx, const float *x, const float *norm_w, float eps, int rows, int K,
                       uint16_t *img, float *rowscale);
+// The embedding rows of `rows` tokens (ids on the device, validated < vocab by
+// the caller) into y, and their RMS-normalised split image.
+int launch_embed_split(cw_ctx *ctx, const float *table, const uint32_t *tok_dev,
+                       const float *norm_w, float eps, int rows, int K, float *y, uint16_t *img,
+                       float *rowscale);
 // *splits = 0 when y was written, else the K splits whose partials are in
 // a.part (a.resid not yet added): [split][M][N], for SwiGLU [split][gate |
 // up][M][N].
@@ -331,9 +360,31 @@ int launch_qk_rope_kv(cw_ctx *ctx, const float *qkv, const float *qn, const floa
                       const float *cos_t, const float *sin_t, int M, int n_heads, int n_kv,
                       int start, int kv_dtype, float *q_out, void *kc, void *vc,
                       const float *part = nullptr, int splits = 0);
-// causal attention of positions start..start+M-1 over an f16 cache, head_dim 128
-int launch_attn_prefill(cw_ctx *ctx, const float *q, const void *kc, const void *vc, int M,
-                        int n_heads, int n_kv, int start, float *out);
+// Causal attention of positions start..start+M-1 over the cache, head_dim 128.
+struct AttnPrefillArgs {
+    const float *q;  // [M][n_heads][128], normalised and rotated
+    const void *kc, *vc;
+    int M, n_heads, n_kv, start;
+    float scale;     // set by launch_attn_prefill
+    int ct;          // set by launch_attn_prefill: key tiles per workgroup
+    float *out;      // one chunk: [M][n_heads][128]
+    float *part;     // more: unnormalised o [chunk][M][n_heads][128], and
+    float *ml;       // (max log2 e, sum) [chunk][M][n_heads]
+};
+struct AttnPrefillPlan {
+    int qt, pt;              // 16-position tiles per wave, positions per workgroup
+    int kt, ct, chunks;      // keys per tile, tiles per chunk, chunks
+    int groups, q_tiles;
+};
+// rows: (chunk, position) rows that part and ml hold
+AttnPrefillPlan attn_prefill_plan(const cw_ctx *ctx, int kv_dtype, int M, int n_heads, int n_kv,
+                                  int start, size_t rows);
+// rows the plan of any prompt of up to M positions takes
+size_t attn_prefill_rows(const cw_ctx *ctx, int M, int n_heads, int n_kv);
+int launch_attn_prefill(cw_ctx *ctx, const AttnPrefillPlan &p, AttnPrefillArgs a, int kv_dtype);
+// The rows' split image for the O projection: of a.out, or of the merged chunks.
+int launch_attn_split(cw_ctx *ctx, const AttnPrefillPlan &p, const AttnPrefillArgs &a,
+                      uint16_t *img, float *rowscale);
 
 // ---- the fused decode step (one persistent cooperative kernel per token)
 

@@ -95,8 +95,9 @@ struct cw_model {
     uint16_t *pf_img = nullptr;    // the current GEMM operand's split image
     float *pf_rowscale = nullptr;  // its per-row powers of two
     uint16_t *pf_spad = nullptr;   // padded scales (matrices that need them)
-    float *pf_part = nullptr;  // split-K partials of the prefill GEMMs
+    float *pf_part = nullptr;  // partials: split-K GEMMs', attention chunks'
     size_t pf_part_floats = 0;
+    size_t pf_attn_rows = 0;   // (chunk, position) rows of attention partials in it
     std::vector<void *> pf_allocs;
 
     // fused decode step (one persistent kernel per token)
@@ -528,7 +529,10 @@ int ensure_prefill(cw_model *m, int n) {
         const int mats = s.epi == EPI_SWIGLU ? 2 : 1;
         spad = std::max(spad, mats * gemm_spad_elems(s.N, s.K, s.s));
     }
-    if (part > 0) CW_TRY(al(part * 4, (void **)&m->pf_part));
+    // ... and the attention chunks' partials
+    m->pf_attn_rows = attn_prefill_rows(m->ctx, n, c.n_heads, c.n_kv_heads);
+    part = std::max(part, m->pf_attn_rows * (m->q_dim + 2 * c.n_heads));
+    CW_TRY(al(part * 4, (void **)&m->pf_part));
     if (spad > 0) CW_TRY(al(spad * 2, (void **)&m->pf_spad));
     m->pf_part_floats = part;
     m->pf_cap = n;
@@ -575,7 +579,6 @@ int tap_row(cw_model *m, float *dst, const float *src, int row, int floats) {
 int enqueue_prefill(cw_model *m, int n, int start) {
     cw_ctx *ctx = m->ctx;
     const auto &c = m->cfg;
-    CW_TRY(launch_embed_rows(ctx, m->embed, c.dim, m->prompt_dev, n, m->pf_hidden));
     const float eps = c.eps;
     // a GEMM's result as the next one's operand, in one pass
     auto to_image = [&](Epi epi, const GemmArgs &a, int splits, const float *norm_w) {
@@ -583,8 +586,21 @@ int enqueue_prefill(cw_model *m, int n, int start) {
     };
     GemmArgs g{};
     int splits = 0;
-    CW_TRY(launch_split_rows(ctx, m->pf_hidden, m->layers[0].attn_norm, eps, n, c.dim, m->pf_img,
-                             m->pf_rowscale));
+    CW_TRY(launch_embed_split(ctx, m->embed, m->prompt_dev, m->layers[0].attn_norm, eps, n, c.dim,
+                              m->pf_hidden, m->pf_img, m->pf_rowscale));
+    const AttnPrefillPlan plan = attn_prefill_plan(ctx, c.kv_dtype, n, c.n_heads, c.n_kv_heads,
+                                                   start, m->pf_attn_rows);
+    AttnPrefillArgs at{};
+    at.q = m->pf_q;
+    at.M = n;
+    at.n_heads = c.n_heads;
+    at.n_kv = c.n_kv_heads;
+    at.start = start;
+    at.out = m->pf_attn;
+    // the chunks' partials share the GEMMs' workspace: those of QKV have been
+    // read when attention starts, those of O are written after the merge
+    at.part = m->pf_part;
+    at.ml = m->pf_part + (size_t)plan.chunks * n * m->q_dim;
     for (int i = 0; i < c.n_layers; ++i) {
         Layer &L = m->layers[i];
         void *kc = (char *)m->kcache + (size_t)i * m->kv_layer_bytes;
@@ -595,10 +611,10 @@ int enqueue_prefill(cw_model *m, int n, int start) {
                                  c.n_heads, c.n_kv_heads, start, c.kv_dtype, m->pf_q, kc, vc,
                                  splits ? m->pf_part : nullptr, splits));
         CW_TRY(tap_row(m, m->tap_q + (size_t)i * m->q_dim, m->pf_q, n - 1, m->q_dim));
-        CW_TRY(launch_attn_prefill(ctx, m->pf_q, kc, vc, n, c.n_heads, c.n_kv_heads, start,
-                                   m->pf_attn));
-        CW_TRY(launch_split_rows(ctx, m->pf_attn, nullptr, eps, n, m->q_dim, m->pf_img,
-                                 m->pf_rowscale));
+        at.kc = kc;
+        at.vc = vc;
+        CW_TRY(launch_attn_prefill(ctx, plan, at, c.kv_dtype));
+        CW_TRY(launch_attn_split(ctx, plan, at, m->pf_img, m->pf_rowscale));
         CW_TRY(pf_gemm(m, n, m->q_dim, EPI_ADD, L.wo, nullptr, m->pf_hidden, m->pf_hidden, &g,
                        &splits));
         CW_TRY(to_image(EPI_ADD, g, splits, L.ffn_norm));
@@ -1153,7 +1169,8 @@ int cw_model_prefill(cw_model *m, const uint32_t *tokens, int n, int start_pos,
         CW_CHECK_ARG(tokens[i] < (uint32_t)c.vocab, "cw_model_prefill: tokens[%d]=%u >= vocab", i,
                      tokens[i]);
     CW_TRY(cw_upload(m->ctx, m->prompt_dev, tokens, (size_t)n * 4));
-    const bool batched = c.kv_dtype == CW_F16 && c.head_dim == 128;
+    // head_dim 128 (either cache type) and more than one position
+    const bool batched = c.head_dim == 128 && n > 1;
     if (batched) {
         CW_TRY(ensure_prefill(m, n));
         CW_TRY(enqueue_prefill(m, n, start_pos));
@@ -1173,7 +1190,7 @@ int cw_model_prefill(cw_model *m, const uint32_t *tokens, int n, int start_pos,
                                      nullptr));
         CW_TRY(launch_rmsnorm(m->ctx, last, m->final_norm, 1, c.dim, c.eps, m->hidden_out));
     } else {
-        // head_dim other than 128 or an f32 cache: the per-token step, n times
+        // another head_dim, or a single token: the per-token step, n times
         GenState s{start_pos, tokens[0], start_pos, n, 0, 0};
         CW_TRY(set_state(m, s));
         CW_TRY(run_steps(m, n, CW_STEP_EAGER));

@@ -8,14 +8,7 @@
 // tiles.
 //
 // Attention must match the f32 per-token path, so no operand is rounded below
-// what the reference computes with: K and V are f16 in the cache and enter f16
-// MFMAs exactly; q and the softmax weights p are split into f16 hi + lo (22
-// significant bits).  The MFMAs accumulate in f32.
-//
-// MFMA v_mfma_f32_16x16x32_f16 (attention): lane l holds A[l % 16][8 (l / 16)
-// + j] and B[8 (l / 16) + j][l % 16] (j = 0..7) and receives
-// D[4 (l / 16) + r][l % 16] (r = 0..3); any k order shared by A and B is
-// valid.
+// what the reference computes with (details at the kernel).
 
 #include <cmath>
 
@@ -25,7 +18,6 @@ namespace {
 
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kT = 256;  // threads per workgroup (4 waves)
 
@@ -61,11 +53,8 @@ __global__ __launch_bounds__(kT) void qk_rope_kv_kernel(const float *__restrict_
     const int q_dim = n_heads * HD, kv_dim = n_kv * HD;
     const size_t row_off = (size_t)i * (q_dim + 2 * kv_dim);
     const float *row = (S > 0 ? part : qkv) + row_off;
-    auto val = [&](const float *p) {  // p: an element of row (of partial 0)
-        float v = *p;
-        for (int s2 = 1; s2 < S; ++s2) v += p[(size_t)s2 * MN];
-        return v;
-    };
+    // p: an element of row (of partial 0)
+    auto val = [&](const float *p) { return S > 0 ? cwi::sum_parts<float>(p, S, MN) : *p; };
     const float c = cos_t[(size_t)pos * HALF + lane], s = sin_t[(size_t)pos * HALF + lane];
     // one head per wave: workgroup y takes heads 4 y .. 4 y + 3 of the row
     for (int h = blockIdx.y * (kT / 64) + wave; h < n_heads + n_kv; h += gridDim.y * (kT / 64)) {
@@ -95,275 +84,319 @@ __global__ __launch_bounds__(kT) void qk_rope_kv_kernel(const float *__restrict_
 }
 
 // ---------------------------------------------------------------------------
-// Causal attention (attention.wgsl:23-96 for each query position) on f16
-// caches, flash style: workgroup = one query head x 64 positions, in two
-// groups of four waves (one wave per 16 positions) that take alternate
-// 64-key tiles, so the longest workgroup runs half as many tile steps.  Per
-// tile: K and V rows staged in LDS as they are stored (16-byte writes);
-// S = q K^T by MFMA (q split into f16 hi/lo), online max / sum per row,
-// P (f16 hi/lo) through LDS into A layout, O += P V by MFMA with the V
-// operand read by LDS transpose loads.  At the end the second group's
-// (max, sum, o) per row merges into the first's through LDS.
-constexpr int kAttQ = 64;   // positions per workgroup
-constexpr int kAttK = 64;   // keys per tile
-constexpr int kKRow = 128 + 8;  // K and V tile row stride (f16), padded
+// Causal attention of M positions (attention.wgsl:23-96 for each) over the
+// cache, flash style.  A workgroup takes one kv head and four waves of query
+// rows: a wave is one query head and QT tiles of 16 positions; the waves are
+// up to four heads of the kv head, then further positions, so that every K / V
+// tile in LDS serves all of them.  It walks key tiles of KT positions, two
+// tiles in LDS (the next one's global -> LDS DMAs in flight), with online
+// max / sum per row.
+//
+// Transposed products keep the softmax in registers: S^T = K q^T leaves lane
+// (g = l / 16, i = l % 16) the keys 4 g + r of query i, which is the B operand
+// of O^T = V^T P^T when the MFMA's k slots are taken in that order (any order
+// shared by A and B is valid).  So P never goes through LDS, and a row's
+// scale is one value per lane.
+//  * f16 cache: v_mfma_f32_16x16x32_f16, K and V as stored, q and P split into
+//    f16 hi + lo (22 significant bits); V^T by LDS transpose loads.
+//  * f32 cache: v_mfma_f32_16x16x4_f32 (lane l: A[l % 16][l / 16],
+//    B[l / 16][l % 16]), every operand f32.
+//
+// Key chunks: a workgroup takes `ct` key tiles of its rows' range, so that few
+// rows against many keys, and the long rows of a causal prompt, still spread
+// over the chip.  With more than one chunk it leaves (max, sum, o) partials,
+// which the pass that reads the rows merges (q4_gemm.hip).
+template <typename KVT, int QT_>
+struct AP {
+    static constexpr int QT = QT_, HD = 128, ES = (int)sizeof(KVT);
+    static constexpr int KT = 128 / ES;        // keys per tile: 16 KB of K
+    static constexpr int ROWB = HD * ES;       // bytes of a cache row slice
+    static constexpr int CPR = ROWB / 16;      // 16-byte chunks per row
+    static constexpr int TILE = KT * ROWB;     // bytes of one K (or V) tile
+    static constexpr int UNITS = TILE / 1024;  // 64-lane DMAs of one tile
+    static constexpr int ST = KT / 16;         // score tiles of 16 keys
+};
 
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+typedef __attribute__((address_space(3))) unsigned char lds_u8;
 
-// B operand of v_mfma_f32_16x16x32_f16 (lane l: B[8 (l / 16) + j][l % 16],
-// j = 0..7) from a row-major LDS tile, B[k][n] = tile[k0 + k][n0 + n].
-// ds_read_b64_tr_b16: within each 16-lane group, lane i receives element
-// i % 4 of the 8 bytes addressed by lane 4 j + i / 4, for j = 0..3.  So lane
-// m of group g addresses row k0 + 8 g + m / 4 (+ 4 for the second read),
-// columns n0 + 4 (m % 4) .. + 3, and lane i gets column n0 + i of rows
-// k0 + 8 g + j.
-__device__ __forceinline__ f16x8 lds_b_tr(const _Float16 *tile, int row_stride, int k0, int n0,
-                                          int lane) {
-    const int g = lane >> 4, m = lane & 15;
-    const _Float16 *p = tile + (size_t)(k0 + 8 * g + (m >> 2)) * row_stride + n0 + 4 * (m & 3);
-    const s16x4 r0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4 *)p);
-    const s16x4 r1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4 *)(p + 4 * row_stride));
-    const uint2 a = __builtin_bit_cast(uint2, r0), b = __builtin_bit_cast(uint2, r1);
-    return __builtin_bit_cast(f16x8, make_uint4(a.x, a.y, b.x, b.y));
+// 64-lane global -> LDS DMA, 16 bytes per lane: lane i's land at lds_dst +
+// 16 i (wave-uniform).  asm, so that the compiler's wait counts leave it out;
+// the kernel waits for it itself.
+__device__ __forceinline__ void dma16(const void *base, uint32_t off, unsigned char *lds_dst) {
+    const uint32_t d = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lds_u8 *)lds_dst);
+    asm volatile("global_load_lds_dwordx4 %0, %1" : : "v"(off), "s"(base), "{m0}"(d) : "memory");
 }
 
-__device__ __forceinline__ uint32_t pack_f16x2(float a, float b) {
-    const uint32_t lo = __builtin_bit_cast(uint16_t, (_Float16)a);
-    const uint32_t hi = __builtin_bit_cast(uint16_t, (_Float16)b);
-    return lo | (hi << 16);
+__device__ __forceinline__ f16x8 pack_f16x8(const float (&v)[8]) {
+    uint32_t p[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+        p[j] = (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)v[2 * j]) |
+               (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)v[2 * j + 1]) << 16;
+    return __builtin_bit_cast(f16x8, make_uint4(p[0], p[1], p[2], p[3]));
 }
 
-constexpr int kAttThreads = 2 * kT;  // two groups of four waves
+// v = hi + lo in f16
+__device__ __forceinline__ void split_f16x8(float (&v)[8], f16x8 &hi, f16x8 &lo) {
+    hi = pack_f16x8(v);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] -= (float)hi[j];
+    lo = pack_f16x8(v);
+}
 
-__global__ __launch_bounds__(kAttThreads) void attn_prefill_kernel(
-    const float *__restrict__ q, const _Float16 *__restrict__ kc, const _Float16 *__restrict__ vc,
-    int M, int n_heads, int n_kv, int start, float scale, float *__restrict__ out) {
-    constexpr int HD = 128;
-    constexpr int TILE = kAttK * kKRow;  // f16 elements of one K (or V) tile
-    // [group][K | V]; after the loop, group 1's (o, m, l) for the merge
-    __shared__ __attribute__((aligned(16))) _Float16 KV[2][2][TILE];
-    __shared__ float Ps[8][16 * kAttK];
-    const int h = blockIdx.x, q0 = blockIdx.y * kAttQ;
+template <typename KVT, int QT, bool PART>
+__global__ __launch_bounds__(kT, 2) void attn_prefill_kernel(cwi::AttnPrefillArgs a) {
+    using C = AP<KVT, QT>;
+    constexpr int HD = C::HD, KT = C::KT, ST = C::ST;
+    constexpr bool F16 = C::ES == 2;
+    __shared__ __attribute__((aligned(1024))) unsigned char lds[2][2 * C::TILE];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int grp = wave >> 2, gw = wave & 3, gtid = tid & (kT - 1);
     const int li = lane & 15, lg = lane >> 4;
-    const int g = h / (n_heads / n_kv);
-    const int kv_dim = n_kv * HD;
-    const int wq = q0 + gw * 16;  // this wave's first position (row of q)
-    _Float16 *Ks = KV[grp][0], *Vs = KV[grp][1];
+    const int hpk = a.n_heads / a.n_kv, hw = hpk < 4 ? hpk : 4;  // heads per workgroup
+    const int h = blockIdx.x * hw + wave % hw, g = h / hpk;
+    // the longest rows first
+    const int qt = gridDim.y - 1 - blockIdx.y;
+    const int pt = QT * 16 * (4 / hw);  // positions per workgroup
+    const int q0 = qt * pt, wq = q0 + wave / hw * (QT * 16);
+    const int last_pos = a.start + min(q0 + pt, a.M) - 1;  // last key any row needs
+    const int t0 = blockIdx.z * a.ct, t1 = min(t0 + a.ct, last_pos / KT + 1);
+    if (t0 >= t1) return;
+    // the last key of this wave's rows (none: rows past M)
+    const int w_last = wq < a.M ? a.start + min(wq + QT * 16, a.M) - 1 : -1;
 
-    // q operands: row li of the wave's 16, dims 8 lg + 32 ks .. +8, hi and lo
-    f16x8 qa[4][2];
-    {
-        const int qi = min(wq + li, M - 1);
-        const float *qr = q + ((size_t)qi * n_heads + h) * HD;
+    const size_t row_b = (size_t)a.n_kv * C::ROWB;
+    const char *const kc = static_cast<const char *>(a.kc) + (size_t)g * C::ROWB;
+    const char *const vc = static_cast<const char *>(a.vc) + (size_t)g * C::ROWB;
+    // Tile t's DMAs: chunk c of row r goes to slot c ^ (r % 16) of its row, so
+    // that both kinds of fragment reads spread over all banks; rows past the
+    // last key re-read it.
+    auto load_tile = [&](int t, unsigned char *buf) {
+        const size_t base = (size_t)t * KT * row_b;
 #pragma unroll
-        for (int ks = 0; ks < 4; ++ks) {
-            const float4 v0 = *reinterpret_cast<const float4 *>(qr + 32 * ks + 8 * lg);
-            const float4 v1 = *reinterpret_cast<const float4 *>(qr + 32 * ks + 8 * lg + 4);
-            const float v[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
-            uint32_t ph[4], pl[4];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const _Float16 a0 = (_Float16)v[2 * j], a1 = (_Float16)v[2 * j + 1];
-                ph[j] = (uint32_t)__builtin_bit_cast(uint16_t, a0) |
-                        ((uint32_t)__builtin_bit_cast(uint16_t, a1) << 16);
-                pl[j] = pack_f16x2(v[2 * j] - (float)a0, v[2 * j + 1] - (float)a1);
-            }
-            qa[ks][0] = __builtin_bit_cast(f16x8, make_uint4(ph[0], ph[1], ph[2], ph[3]));
-            qa[ks][1] = __builtin_bit_cast(f16x8, make_uint4(pl[0], pl[1], pl[2], pl[3]));
-        }
-    }
-
-    // rows of this lane in the C layout: 4 lg + r of the wave's 16
-    float mrow[4], lrow[4];
-    f32x4 o[8];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        mrow[r] = -INFINITY;
-        lrow[r] = 0.0f;
-    }
-#pragma unroll
-    for (int ni = 0; ni < 8; ++ni) o[ni] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-    const int last_pos = start + min(q0 + kAttQ, M) - 1;  // last key any row needs
-    const int n_tiles = last_pos / kAttK + 1;
-    const int n_steps = (n_tiles + 1) / 2;  // group grp takes tiles grp, grp + 2, ...
-    // K and V rows of key tile t, 64 keys x 128 dims, 16 B per load (4 each
-    // per thread of the group); the group's next tile's loads are in flight
-    // during this tile's MFMAs (past the last tile a clamped re-load, unused)
-    u32x4 kn[4], vn[4];
-    auto tile_load = [&](int t) {
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int f = gtid + u * kT;  // 0..1023
-            const int key = f >> 4, c8 = (f & 15) * 8;
-            const int p = min(t * kAttK + key, last_pos);
-            kn[u] = *reinterpret_cast<const u32x4 *>(kc + (size_t)p * kv_dim + g * HD + c8);
-            vn[u] = *reinterpret_cast<const u32x4 *>(vc + (size_t)p * kv_dim + g * HD + c8);
+        for (int p = 0; p < C::UNITS / 4; ++p) {
+            const int u = wave + p * 4;
+            const int r = u * (64 / C::CPR) + lane / C::CPR;
+            const int c = (lane % C::CPR) ^ (r & 15);
+            const uint32_t off = (uint32_t)min(r, last_pos - t * KT) * (uint32_t)row_b + c * 16;
+            dma16(kc + base, off, buf + u * 1024);
+            dma16(vc + base, off, buf + C::TILE + u * 1024);
         }
     };
-    tile_load(min(grp, n_tiles - 1));
-    for (int st = 0; st < n_steps; ++st) {
-        const int t = 2 * st + grp;
-        const bool active = t < n_tiles;  // (uniform over the group)
-        const int k0 = t * kAttK;
-        __syncthreads();  // previous step's LDS reads are done
-        // stage K and V rows
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int f = gtid + u * kT;
-            const int key = f >> 4, c8 = (f & 15) * 8;
-            *reinterpret_cast<u32x4 *>(&Ks[key * kKRow + c8]) = kn[u];
-            *reinterpret_cast<u32x4 *>(&Vs[key * kKRow + c8]) = vn[u];
-        }
-        tile_load(min(t + 2, n_tiles - 1));
-        __builtin_amdgcn_sched_barrier(0);
-        __syncthreads();
-        if (!active) continue;
+    load_tile(t0, lds[0]);
 
-        // S (16 rows x 64 keys): 4 key tiles of 16, K = 128 dims in 4 steps
-        f32x4 sc[4];
+    // q operands of this lane's queries (B: query li, dims in the k order of
+    // the K fragments), times scale log2(e): p = 2^(s - max)
+    f16x8 qh[F16 ? QT : 1][4], ql[F16 ? QT : 1][4];
+    f32x4 qf[F16 ? 1 : QT][8];
 #pragma unroll
-        for (int ni = 0; ni < 4; ++ni) {
-            f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < QT; ++i) {
+        const float *qr = a.q + ((size_t)min(wq + i * 16 + li, a.M - 1) * a.n_heads + h) * HD;
+        if constexpr (F16) {
 #pragma unroll
             for (int ks = 0; ks < 4; ++ks) {
-                const f16x8 kb = *reinterpret_cast<const f16x8 *>(
-                    &Ks[(ni * 16 + li) * kKRow + 32 * ks + 8 * lg]);
-                acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(qa[ks][0], kb, acc, 0, 0, 0);
-                acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(qa[ks][1], kb, acc, 0, 0, 0);
+                const float4 v0 = *reinterpret_cast<const float4 *>(qr + 32 * ks + 8 * lg);
+                const float4 v1 = *reinterpret_cast<const float4 *>(qr + 32 * ks + 8 * lg + 4);
+                float v[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
+                split_f16x8(v, qh[i][ks], ql[i][ks]);
             }
-            sc[ni] = acc;
+        } else {
+#pragma unroll
+            for (int u = 0; u < 8; ++u)
+                qf[i][u] = *reinterpret_cast<const f32x4 *>(qr + 16 * u + 4 * lg);
         }
-        // mask (causal, and rows past M), scale, online softmax per row
-        float pm[4][4];
+    }
+
+    f32x4 o[QT][8];  // O^T: dims 16 d + 4 lg + r of query li
+    float mrow[QT], lsum[QT];  // running max (times log2 e); this lane's part of the sum
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int row_pos = start + wq + 4 * lg + r;
-            float mx = -INFINITY;
+    for (int i = 0; i < QT; ++i) {
+        mrow[i] = -INFINITY;
+        lsum[i] = 0.0f;
 #pragma unroll
-            for (int ni = 0; ni < 4; ++ni) {
-                const int key = k0 + ni * 16 + li;
-                const float v = key <= row_pos ? sc[ni][r] * scale : -INFINITY;
-                pm[ni][r] = v;
-                mx = fmaxf(mx, v);
+        for (int d = 0; d < 8; ++d) o[i][d] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    // fragment addresses within a tile; other k steps (dims) by xor, other
+    // rows by a constant
+    const int ka = li * C::ROWB + ((lg ^ li) << 4);
+    const int va = F16 ? (4 * lg + (li >> 2)) * C::ROWB +
+                             ((((li & 3) >> 1) ^ (4 * lg + (li >> 2))) << 4) + (li & 1) * 8
+                       : 0;
+
+    for (int t = t0; t < t1; ++t) {
+        unsigned char *const buf = lds[(t - t0) & 1];
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's part of tile t has landed
+        __builtin_amdgcn_sched_barrier(0);
+        __atomic_signal_fence(__ATOMIC_SEQ_CST);
+        __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+        __builtin_amdgcn_s_barrier();        // tile t published; the other buffer is free
+        __atomic_signal_fence(__ATOMIC_SEQ_CST);
+        if (t + 1 < t1) load_tile(t + 1, lds[(t - t0 + 1) & 1]);
+        const int k0 = t * KT;
+        if (k0 > w_last) continue;  // (wave-uniform) every key is past this wave's rows
+        const unsigned char *const Ks = buf, *const Vs = buf + C::TILE;
+
+        f32x4 s[QT][ST];
+#pragma unroll
+        for (int kt = 0; kt < ST; ++kt) {
+#pragma unroll
+            for (int i = 0; i < QT; ++i) s[i][kt] = f32x4{0.f, 0.f, 0.f, 0.f};
+            if constexpr (F16) {
+#pragma unroll
+                for (int ks = 0; ks < 4; ++ks) {
+                    const f16x8 kf = *reinterpret_cast<const f16x8 *>(
+                        Ks + ((ka ^ (ks << 6)) + kt * 16 * C::ROWB));
+#pragma unroll
+                    for (int i = 0; i < QT; ++i)
+                        s[i][kt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, qh[i][ks], s[i][kt],
+                                                                          0, 0, 0);
+#pragma unroll
+                    for (int i = 0; i < QT; ++i)
+                        s[i][kt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, ql[i][ks], s[i][kt],
+                                                                          0, 0, 0);
+                }
+            } else {
+#pragma unroll
+                for (int u = 0; u < 8; ++u) {
+                    const f32x4 kf = *reinterpret_cast<const f32x4 *>(
+                        Ks + ((ka ^ (u << 6)) + kt * 16 * C::ROWB));
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+#pragma unroll
+                        for (int i = 0; i < QT; ++i)
+                            s[i][kt] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[r], qf[i][u][r],
+                                                                            s[i][kt], 0, 0, 0);
+                }
             }
-            // max over the 16 lanes that share this row (same lg)
+        }
+        // online softmax of each query; keys past its position only in tiles
+        // that reach beyond the wave's first row
+        float alpha[QT];
+        bool grew = false;
 #pragma unroll
-            for (int off = 8; off >= 1; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off));
-            const float mnew = fmaxf(mrow[r], mx);
-            // a row with no key yet keeps mnew = -inf: guard the rescale
-            const float alpha = mnew == -INFINITY ? 1.0f : expf(mrow[r] - mnew);
+        for (int i = 0; i < QT; ++i) {
+            const int lim = a.start + wq + i * 16 + li - k0 - 4 * lg;  // last key: 16 kt + r
+            if (k0 + KT - 1 > a.start + wq + i * 16) {
+#pragma unroll
+                for (int kt = 0; kt < ST; ++kt)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        s[i][kt][r] = kt * 16 + r <= lim ? s[i][kt][r] : -INFINITY;
+            }
+            float mx = s[i][0][0];
+#pragma unroll
+            for (int kt = 0; kt < ST; ++kt)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) mx = fmaxf(mx, s[i][kt][r]);
+            mx = fmaxf(mx, __shfl_xor(mx, 16));
+            mx = fmaxf(mx, __shfl_xor(mx, 32));
+            const float mnew = fmaxf(mrow[i], mx * a.scale);
+            // a query with no key yet keeps max -inf: its terms are 2^-inf = 0
+            const float ref = mnew == -INFINITY ? 0.0f : mnew;
+            alpha[i] = __builtin_amdgcn_exp2f(mrow[i] - ref);
+            grew |= mnew > mrow[i];
+            mrow[i] = mnew;
             float ls = 0.0f;
 #pragma unroll
-            for (int ni = 0; ni < 4; ++ni) {
-                const float p = pm[ni][r] == -INFINITY ? 0.0f : expf(pm[ni][r] - mnew);
-                pm[ni][r] = p;
-                ls += p;
-            }
+            for (int kt = 0; kt < ST; ++kt)
 #pragma unroll
-            for (int off = 8; off >= 1; off >>= 1) ls += __shfl_xor(ls, off);
-            lrow[r] = lrow[r] * alpha + ls;
-            mrow[r] = mnew;
-#pragma unroll
-            for (int ni = 0; ni < 8; ++ni) o[ni][r] *= alpha;
+                for (int r = 0; r < 4; ++r) {
+                    const float p =
+                        __builtin_amdgcn_exp2f(__builtin_fmaf(s[i][kt][r], a.scale, -ref));
+                    s[i][kt][r] = p;
+                    ls += p;
+                }
+            lsum[i] = lsum[i] * alpha[i] + ls;
         }
-        // P to LDS (row-major 16 x 64), back in A layout as f16 hi/lo
-        float *P = Ps[wave];
+        if (__any(grew)) {
 #pragma unroll
-        for (int ni = 0; ni < 4; ++ni)
+            for (int i = 0; i < QT; ++i)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) P[(4 * lg + r) * kAttK + ni * 16 + li] = pm[ni][r];
-        // (a wave's LDS accesses complete in order: its reads below see these writes)
-        f16x8 pa[2][2];
+                for (int d = 0; d < 8; ++d)
 #pragma unroll
-        for (int kk = 0; kk < 2; ++kk) {
-            const float *pr = P + li * kAttK + 32 * kk + 8 * lg;
-            uint32_t ph[4], pl[4];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const float v0 = pr[2 * j], v1 = pr[2 * j + 1];
-                const _Float16 a0 = (_Float16)v0, a1 = (_Float16)v1;
-                ph[j] = (uint32_t)__builtin_bit_cast(uint16_t, a0) |
-                        ((uint32_t)__builtin_bit_cast(uint16_t, a1) << 16);
-                pl[j] = pack_f16x2(v0 - (float)a0, v1 - (float)a1);
-            }
-            pa[kk][0] = __builtin_bit_cast(f16x8, make_uint4(ph[0], ph[1], ph[2], ph[3]));
-            pa[kk][1] = __builtin_bit_cast(f16x8, make_uint4(pl[0], pl[1], pl[2], pl[3]));
+                    for (int r = 0; r < 4; ++r) o[i][d][r] *= alpha[i];
         }
-        // O (16 rows x 128 dims) += P (16 x 64 keys) V (64 keys x 128 dims)
+        if constexpr (F16) {
 #pragma unroll
-        for (int ni = 0; ni < 8; ++ni) {
+            for (int kk = 0; kk < ST / 2; ++kk) {
+                f16x8 ph[QT], pl[QT];
 #pragma unroll
-            for (int kk = 0; kk < 2; ++kk) {
-                const f16x8 vb = lds_b_tr(Vs, kKRow, 32 * kk, ni * 16, lane);
-                o[ni] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pa[kk][0], vb, o[ni], 0, 0, 0);
-                o[ni] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pa[kk][1], vb, o[ni], 0, 0, 0);
+                for (int i = 0; i < QT; ++i) {
+                    float v[8];
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        v[r] = s[i][2 * kk][r];
+                        v[4 + r] = s[i][2 * kk + 1][r];
+                    }
+                    split_f16x8(v, ph[i], pl[i]);
+                }
+#pragma unroll
+                for (int d = 0; d < 8; ++d) {
+                    // ds_read_b64_tr_b16: within each 16-lane group, lane i
+                    // receives element i % 4 of the 8 bytes addressed by lane
+                    // 4 j + i / 4, for j = 0..3: dim 16 d + i of keys 4 lg + j
+                    const unsigned char *p = Vs + ((va ^ (d << 5)) + kk * 32 * C::ROWB);
+                    const uint2 r0 = __builtin_bit_cast(
+                        uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4 *)p));
+                    const uint2 r1 = __builtin_bit_cast(
+                        uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                                   (lds_s16x4 *)(p + 16 * C::ROWB)));
+                    const f16x8 vf =
+                        __builtin_bit_cast(f16x8, make_uint4(r0.x, r0.y, r1.x, r1.y));
+#pragma unroll
+                    for (int i = 0; i < QT; ++i)
+                        o[i][d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf, ph[i], o[i][d], 0, 0, 0);
+#pragma unroll
+                    for (int i = 0; i < QT; ++i)
+                        o[i][d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf, pl[i], o[i][d], 0, 0, 0);
+                }
             }
+        } else {
+#pragma unroll
+            for (int kt = 0; kt < ST; ++kt)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int row = 4 * lg + r;
+                    const int vb = row * C::ROWB + (((li >> 2) ^ row) << 4) + (li & 3) * 4;
+#pragma unroll
+                    for (int d = 0; d < 8; ++d) {
+                        const float vf = *reinterpret_cast<const float *>(
+                            Vs + ((vb ^ (d << 6)) + kt * 16 * C::ROWB));
+#pragma unroll
+                        for (int i = 0; i < QT; ++i)
+                            o[i][d] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf, s[i][kt][r], o[i][d],
+                                                                           0, 0, 0);
+                    }
+                }
         }
     }
 
-    // merge: group 1's (o, m, l) of each row through LDS into group 0's
-    // (rescaled to the common max), then normalise and store.  Lane holds
-    // rows 4 lg + r, dims ni * 16 + li.
-    __syncthreads();  // every group is done with its K / V tile
-    float *mo = reinterpret_cast<float *>(&KV[0][0][0]);  // [4 waves][16 rows][128]
-    float *mml = mo + 4 * 16 * HD;                        // [4 waves][16 rows][2]
-    if (grp == 1) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int row = 4 * lg + r;
+    for (int i = 0; i < QT; ++i) {
+        float l = lsum[i];
+        l += __shfl_xor(l, 16);
+        l += __shfl_xor(l, 32);
+        const int qi = wq + i * 16 + li;
+        if (qi >= a.M) continue;
+        const size_t row = (size_t)qi * a.n_heads + h;
+        const size_t prow = (size_t)blockIdx.z * a.M * a.n_heads + row;
+        float *dst = PART ? a.part + prow * HD : a.out + row * HD;
+        const float f = PART ? 1.0f : 1.0f / l;
 #pragma unroll
-            for (int ni = 0; ni < 8; ++ni) mo[(gw * 16 + row) * HD + ni * 16 + li] = o[ni][r];
-            if (li == 0) {
-                mml[(gw * 16 + row) * 2] = mrow[r];
-                mml[(gw * 16 + row) * 2 + 1] = lrow[r];
-            }
-        }
+        for (int d = 0; d < 8; ++d)
+            *reinterpret_cast<float4 *>(dst + 16 * d + 4 * lg) =
+                make_float4(o[i][d][0] * f, o[i][d][1] * f, o[i][d][2] * f, o[i][d][3] * f);
+        if (PART && lg == 0)
+            *reinterpret_cast<float2 *>(a.ml + prow * 2) = make_float2(mrow[i], l);
     }
-    __syncthreads();
-    if (grp == 0) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int row = 4 * lg + r;
-            const int qi = wq + row;
-            const float m1 = mml[(gw * 16 + row) * 2], l1 = mml[(gw * 16 + row) * 2 + 1];
-            const float mm = fmaxf(mrow[r], m1);
-            const float f0 = mrow[r] == -INFINITY ? 0.0f : expf(mrow[r] - mm);
-            const float f1 = m1 == -INFINITY ? 0.0f : expf(m1 - mm);
-            const float inv = 1.0f / (lrow[r] * f0 + l1 * f1);
-            if (qi < M) {
-                float *dst = out + (size_t)qi * n_heads * HD + (size_t)h * HD;
-#pragma unroll
-                for (int ni = 0; ni < 8; ++ni)
-                    dst[ni * 16 + li] =
-                        (o[ni][r] * f0 + mo[(gw * 16 + row) * HD + ni * 16 + li] * f1) * inv;
-            }
-        }
-    }
-}
-
-// Embedding rows of n tokens (Qwen3::embed, qwen3.rs:128-133): one workgroup
-// per position.
-__global__ __launch_bounds__(kT) void embed_rows_kernel(const float *__restrict__ table, int dim,
-                                                        const uint32_t *__restrict__ tok,
-                                                        float *__restrict__ out) {
-    const size_t src = (size_t)tok[blockIdx.x] * dim, dst = (size_t)blockIdx.x * dim;
-    for (int i = threadIdx.x; i < dim; i += kT) out[dst + i] = table[src + i];
 }
 
 }  // namespace
 
 namespace cwi {
-
-int launch_embed_rows(cw_ctx *ctx, const float *table, int dim, const uint32_t *tok_dev, int n,
-                      float *out) {
-    return launch(ctx, "prefill_embed", embed_rows_kernel, dim3(n), dim3(kT), 0, table, dim,
-                  tok_dev, out);
-}
 
 int launch_qk_rope_kv(cw_ctx *ctx, const float *qkv, const float *qn, const float *kn, float eps,
                       const float *cos_t, const float *sin_t, int M, int n_heads, int n_kv,
@@ -381,12 +414,60 @@ int launch_qk_rope_kv(cw_ctx *ctx, const float *qkv, const float *qn, const floa
                   part, S, mn);
 }
 
-int launch_attn_prefill(cw_ctx *ctx, const float *q, const void *kc, const void *vc, int M,
-                        int n_heads, int n_kv, int start, float *out) {
-    const float scale = 1.0f / sqrtf(128.0f);
-    return launch(ctx, "prefill_attention", attn_prefill_kernel,
-                  dim3(n_heads, (M + kAttQ - 1) / kAttQ), dim3(kAttThreads), 0, q,
-                  (const _Float16 *)kc, (const _Float16 *)vc, M, n_heads, n_kv, start, scale, out);
+// Positions per workgroup of one query tile, and the tiles of keys per
+// workgroup: the share of all (query tile, key tile) steps that two
+// workgroups per CU take, so no workgroup runs longer than that.  `rows`: the
+// most (chunk, position) partials there is room for.
+AttnPrefillPlan attn_prefill_plan(const cw_ctx *ctx, int kv_dtype, int M, int n_heads, int n_kv,
+                                  int start, size_t rows) {
+    const int hpk = n_heads / n_kv, hw = std::min(hpk, 4);
+    AttnPrefillPlan p{};
+    // two query tiles per wave read each K / V fragment once for both; one
+    // when the rows fill no more, and for f32, whose MFMAs outweigh the reads
+    // (and whose second tile would not fit the registers)
+    p.qt = M <= 16 * (4 / hw) || kv_dtype != CW_F16 ? 1 : 2;
+    p.pt = p.qt * 16 * (4 / hw);
+    p.kt = kv_dtype == CW_F16 ? AP<_Float16, 1>::KT : AP<float, 1>::KT;
+    p.groups = n_heads / hw;
+    p.q_tiles = (M + p.pt - 1) / p.pt;
+    long steps = 0;
+    for (int t = 0; t < p.q_tiles; ++t)
+        steps += (start + std::min((t + 1) * p.pt, M) - 1) / p.kt + 1;
+    const int tiles = (start + M - 1) / p.kt + 1;
+    const long slots = 2L * ctx->n_cu;
+    p.ct = (int)((steps * p.groups + slots - 1) / slots);
+    p.chunks = (tiles + p.ct - 1) / p.ct;
+    if ((size_t)p.chunks * M > rows) {
+        p.chunks = (int)std::max<size_t>(1, rows / M);
+        p.ct = (tiles + p.chunks - 1) / p.chunks;
+        p.chunks = (tiles + p.ct - 1) / p.ct;
+    }
+    return p;
+}
+
+size_t attn_prefill_rows(const cw_ctx *ctx, int M, int n_heads, int n_kv) {
+    // chunks <= 2 slots / (groups q_tiles) + 1 (a causal row range is at least
+    // half of the longest), and q_tiles >= M / pt
+    const int hw = std::min(n_heads / n_kv, 4), groups = n_heads / hw;
+    return (size_t)M + (size_t)4 * ctx->n_cu * 32 * (4 / hw) / groups + 1;
+}
+
+int launch_attn_prefill(cw_ctx *ctx, const AttnPrefillPlan &p, AttnPrefillArgs a, int kv_dtype) {
+    // p = 2^(s scale log2(e) - max)
+    a.scale = (float)(1.4426950408889634 / sqrt(128.0));
+    a.ct = p.ct;
+    const dim3 grid(p.groups, p.q_tiles, p.chunks);
+    auto go = [&](auto fn) { return launch(ctx, "prefill_attention", fn, grid, dim3(kT), 0, a); };
+    const bool part = p.chunks > 1;
+    if (kv_dtype == CW_F16) {
+        if (p.qt == 1)
+            return part ? go(attn_prefill_kernel<_Float16, 1, true>)
+                        : go(attn_prefill_kernel<_Float16, 1, false>);
+        return part ? go(attn_prefill_kernel<_Float16, 2, true>)
+                    : go(attn_prefill_kernel<_Float16, 2, false>);
+    }
+    return part ? go(attn_prefill_kernel<float, 1, true>)
+                : go(attn_prefill_kernel<float, 1, false>);
 }
 
 }  // namespace cwi

@@ -54,43 +54,28 @@ constexpr float kUnscale = 0.0625f;  // the products' factor 16
 // One workgroup per row; a thread takes whole chunks (8 elements), CH of them
 // in registers.  Sources of a row: SRC_ROWS, x itself; SRC_PART, the sum in
 // order of S split-K partials (+ resid), also written to y; SRC_SWIGLU,
-// silu(g) u of the summed partials of the gate and the up product.  NORM:
-// RMSNorm first (norm.wgsl:20-42).
-enum SplitSrc { SRC_ROWS, SRC_PART, SRC_SWIGLU };
+// silu(g) u of the summed partials of the gate and the up product; SRC_EMBED,
+// a token's embedding row (Qwen3::embed, qwen3.rs:128-133), also written to y;
+// SRC_ATTN, the attention chunks of a position merged.  NORM: RMSNorm first
+// (norm.wgsl:20-42).
+enum SplitSrc { SRC_ROWS, SRC_PART, SRC_SWIGLU, SRC_EMBED, SRC_ATTN };
 
 struct SplitArgs {
-    const float *x;       // [M][K], or the partials [S][M][K] ([S][2][M][K])
+    const float *x;       // [M][K], the partials [S][M][K] ([S][2][M][K]), the table
     int S;
     size_t MK;            // elements of one [M][K] matrix
     const float *resid;   // SRC_PART, optional: [M][K]
-    float *y;             // SRC_PART: [M][K]
+    float *y;             // SRC_PART, SRC_EMBED: [M][K]
+    const uint32_t *tok;  // SRC_EMBED
+    const float *ml;      // SRC_ATTN: (max log2 e, sum) [S][M][K / 128]
+    int M, start, pt, span;  // SRC_ATTN: rows, first position, positions that
+                             // share their chunks, positions per chunk
     const float *norm_w;  // NORM: gain [K]
     float eps;
     int K;
     uint16_t *img;
     float *rowscale;
 };
-
-// The sum in order of partials p[0], p[stride], .. p[(S - 1) stride]: eight
-// requested at a time, so that no load waits for another's sum.
-__device__ __forceinline__ float4 sum_parts(const float *p, int S, size_t stride) {
-    float4 v = *reinterpret_cast<const float4 *>(p);
-    for (int s = 1; s < S; s += 8) {
-        float4 t[8];
-#pragma unroll
-        for (int u = 0; u < 8; ++u)
-            t[u] = *reinterpret_cast<const float4 *>(p + (size_t)min(s + u, S - 1) * stride);
-#pragma unroll
-        for (int u = 0; u < 8; ++u)
-            if (s + u < S) {
-                v.x += t[u].x;
-                v.y += t[u].y;
-                v.z += t[u].z;
-                v.w += t[u].w;
-            }
-    }
-    return v;
-}
 
 __device__ __forceinline__ float silu_mul(float g, float u) { return g / (1.0f + expf(-g)) * u; }
 
@@ -100,28 +85,70 @@ __global__ __launch_bounds__(512) void split_image_kernel(SplitArgs a) {
     const int tid = threadIdx.x, nt = blockDim.x, lane = tid & 63, wave = tid >> 6;
     const int nch = a.K >> 3;  // chunks of the row
     const size_t base = (size_t)blockIdx.x * a.K;
-    auto load4 = [&](size_t o) {
-        if constexpr (SRC == SRC_ROWS) return *reinterpret_cast<const float4 *>(a.x + o);
-        if constexpr (SRC == SRC_SWIGLU) {
-            const float4 g = sum_parts(a.x + o, a.S, 2 * a.MK);
-            const float4 u = sum_parts(a.x + a.MK + o, a.S, 2 * a.MK);
-            return make_float4(silu_mul(g.x, u.x), silu_mul(g.y, u.y), silu_mul(g.z, u.z),
-                               silu_mul(g.w, u.w));
+    // elements 4 g .. of the block and 16 + 4 g .. for chunk c
+    auto load8 = [&](int c, float4 &ve, float4 &vf) {
+        const size_t col = (size_t)(c >> 2) * 32 + 4 * (c & 3), o = base + col;
+        if constexpr (SRC == SRC_ROWS || SRC == SRC_EMBED) {
+            const float *p = a.x + (SRC == SRC_EMBED ? (size_t)a.tok[blockIdx.x] * a.K + col : o);
+            ve = *reinterpret_cast<const float4 *>(p);
+            vf = *reinterpret_cast<const float4 *>(p + 16);
+        } else if constexpr (SRC == SRC_SWIGLU) {
+            float4 v[2];
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+                const float4 g = cwi::sum_parts<float4>(a.x + o + 16 * k, a.S, 2 * a.MK);
+                const float4 u = cwi::sum_parts<float4>(a.x + a.MK + o + 16 * k, a.S, 2 * a.MK);
+                v[k] = make_float4(silu_mul(g.x, u.x), silu_mul(g.y, u.y), silu_mul(g.z, u.z),
+                                   silu_mul(g.w, u.w));
+            }
+            ve = v[0];
+            vf = v[1];
+        } else if constexpr (SRC == SRC_ATTN) {
+            // the chunks that reach the last key of this position's tile
+            const int last = a.start + min(((int)blockIdx.x / a.pt + 1) * a.pt, a.M) - 1;
+            const int n = last / a.span + 1;
+            const size_t heads = a.K / 128, step = (size_t)a.M * heads;
+            const float2 *ml = reinterpret_cast<const float2 *>(a.ml) + blockIdx.x * heads +
+                               col / 128;
+            float m = -INFINITY, l = 0.0f;
+            for (int i = 0; i < n; ++i) m = fmaxf(m, ml[i * step].x);
+            ve = vf = make_float4(0.f, 0.f, 0.f, 0.f);
+            for (int i = 0; i < n; ++i) {
+                const float2 p = ml[i * step];
+                const float f = __builtin_amdgcn_exp2f(p.x - m);
+                const float4 e = *reinterpret_cast<const float4 *>(a.x + i * a.MK + o);
+                const float4 h = *reinterpret_cast<const float4 *>(a.x + i * a.MK + o + 16);
+                l = __builtin_fmaf(f, p.y, l);
+                ve.x = __builtin_fmaf(f, e.x, ve.x);
+                ve.y = __builtin_fmaf(f, e.y, ve.y);
+                ve.z = __builtin_fmaf(f, e.z, ve.z);
+                ve.w = __builtin_fmaf(f, e.w, ve.w);
+                vf.x = __builtin_fmaf(f, h.x, vf.x);
+                vf.y = __builtin_fmaf(f, h.y, vf.y);
+                vf.z = __builtin_fmaf(f, h.z, vf.z);
+                vf.w = __builtin_fmaf(f, h.w, vf.w);
+            }
+            const float r = 1.0f / l;
+            ve = make_float4(ve.x * r, ve.y * r, ve.z * r, ve.w * r);
+            vf = make_float4(vf.x * r, vf.y * r, vf.z * r, vf.w * r);
+        } else {
+            float4 v[2];
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+                v[k] = cwi::sum_parts<float4>(a.x + o + 16 * k, a.S, a.MK);
+                if (a.resid) {
+                    const float4 r = *reinterpret_cast<const float4 *>(a.resid + o + 16 * k);
+                    v[k] = make_float4(r.x + v[k].x, r.y + v[k].y, r.z + v[k].z, r.w + v[k].w);
+                }
+            }
+            ve = v[0];
+            vf = v[1];
         }
-        float4 v = sum_parts(a.x + o, a.S, a.MK);
-        if (a.resid) {
-            const float4 r = *reinterpret_cast<const float4 *>(a.resid + o);
-            v.x = r.x + v.x;
-            v.y = r.y + v.y;
-            v.z = r.z + v.z;
-            v.w = r.w + v.w;
-        }
-        return v;
     };
     float ss = 0.0f, mx = 0.0f;
     auto scan = [&](int c, float4 ve, float4 vf) {
         const int o = (c >> 2) * 32 + 4 * (c & 3);
-        if constexpr (SRC == SRC_PART) {
+        if constexpr (SRC == SRC_PART || SRC == SRC_EMBED) {
             *reinterpret_cast<float4 *>(a.y + base + o) = ve;
             *reinterpret_cast<float4 *>(a.y + base + o + 16) = vf;
         }
@@ -144,20 +171,16 @@ __global__ __launch_bounds__(512) void split_image_kernel(SplitArgs a) {
     };
     // the first CH chunks of a thread stay in registers; a longer row's rest
     // is read again for the second pass
-    float4 ve[CH], vf[CH];  // elements 4 g .. of the block, and 16 + 4 g ..
+    float4 ve[CH], vf[CH];
 #pragma unroll
-    for (int j = 0; j < CH; ++j) {
-        const int c = min(tid + j * nt, nch - 1);
-        const size_t o = base + (size_t)(c >> 2) * 32 + 4 * (c & 3);
-        ve[j] = load4(o);
-        vf[j] = load4(o + 16);
-    }
+    for (int j = 0; j < CH; ++j) load8(min(tid + j * nt, nch - 1), ve[j], vf[j]);
 #pragma unroll
     for (int j = 0; j < CH; ++j)
         if (tid + j * nt < nch) scan(tid + j * nt, ve[j], vf[j]);
     for (int c = tid + CH * nt; c < nch; c += nt) {
-        const size_t o = base + (size_t)(c >> 2) * 32 + 4 * (c & 3);
-        scan(c, load4(o), load4(o + 16));
+        float4 e, f;
+        load8(c, e, f);
+        scan(c, e, f);
     }
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) {
@@ -209,12 +232,15 @@ __global__ __launch_bounds__(512) void split_image_kernel(SplitArgs a) {
     for (int j = 0; j < CH; ++j)
         if (tid + j * nt < nch) emit(tid + j * nt, ve[j], vf[j]);
     for (int c = tid + CH * nt; c < nch; c += nt) {
-        const size_t o = base + (size_t)(c >> 2) * 32 + 4 * (c & 3);
-        if constexpr (SRC == SRC_PART)  // this thread's own stores
-            emit(c, *reinterpret_cast<const float4 *>(a.y + o),
-                 *reinterpret_cast<const float4 *>(a.y + o + 16));
-        else
-            emit(c, load4(o), load4(o + 16));
+        float4 e, f;
+        if constexpr (SRC == SRC_PART) {  // this thread's own stores
+            const size_t o = base + (size_t)(c >> 2) * 32 + 4 * (c & 3);
+            e = *reinterpret_cast<const float4 *>(a.y + o);
+            f = *reinterpret_cast<const float4 *>(a.y + o + 16);
+        } else {
+            load8(c, e, f);
+        }
+        emit(c, e, f);
     }
 }
 
@@ -226,7 +252,7 @@ __global__ __launch_bounds__(kT) void gemm_reduce_kernel(const float *__restrict
     const bool vec = n % 4 == 0 && ((reinterpret_cast<uintptr_t>(y) |
                                      reinterpret_cast<uintptr_t>(resid)) & 15) == 0;
     if (vec) {
-        float4 v = sum_parts(part + i, S, n);
+        float4 v = cwi::sum_parts<float4>(part + i, S, n);
         if (resid) {
             const float4 r = *reinterpret_cast<const float4 *>(resid + i);
             v.x = r.x + v.x;
@@ -718,6 +744,39 @@ int launch_split_rows(cw_ctx *ctx, const float *x, const float *norm_w, float ep
     a.rowscale = rowscale;
     return norm_w ? launch_split_image<true, SRC_ROWS>(ctx, "prefill_split_rmsnorm", a, rows)
                   : launch_split_image<false, SRC_ROWS>(ctx, "prefill_split", a, rows);
+}
+
+int launch_embed_split(cw_ctx *ctx, const float *table, const uint32_t *tok_dev,
+                       const float *norm_w, float eps, int rows, int K, float *y, uint16_t *img,
+                       float *rowscale) {
+    SplitArgs a{};
+    a.x = table;
+    a.tok = tok_dev;
+    a.y = y;
+    a.norm_w = norm_w;
+    a.eps = eps;
+    a.K = K;
+    a.img = img;
+    a.rowscale = rowscale;
+    return launch_split_image<true, SRC_EMBED>(ctx, "prefill_embed_split", a, rows);
+}
+
+int launch_attn_split(cw_ctx *ctx, const AttnPrefillPlan &p, const AttnPrefillArgs &t,
+                      uint16_t *img, float *rowscale) {
+    const int K = t.n_heads * 128;
+    if (p.chunks == 1) return launch_split_rows(ctx, t.out, nullptr, 0.0f, t.M, K, img, rowscale);
+    SplitArgs a{};
+    a.x = t.part;
+    a.MK = (size_t)t.M * K;
+    a.ml = t.ml;
+    a.M = t.M;
+    a.start = t.start;
+    a.pt = p.pt;
+    a.span = p.ct * p.kt;
+    a.K = K;
+    a.img = img;
+    a.rowscale = rowscale;
+    return launch_split_image<false, SRC_ATTN>(ctx, "prefill_attention_merge", a, t.M);
 }
 
 int launch_q4_gemm(cw_ctx *ctx, Epi epi, GemmArgs a, int *splits) {

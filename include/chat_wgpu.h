@@ -316,8 +316,8 @@ int cw_step_dry_plan(const cw_model_config *cfg, int n_cu, int split_gate_up, vo
 /* The prompt phase of model::generate (src/model/mod.rs:57-125: P forwards,
  * the logits of all but the last discarded) for n tokens at positions
  * start_pos..start_pos+n-1, batched: each layer runs as Q4_0 GEMMs on the
- * matrix cores and causal attention over the cache (f16 cache and head_dim
- * 128; other configurations run the per-token step n times).  Writes the KV
+ * matrix cores and causal attention over the cache (head_dim 128 and n > 1;
+ * otherwise the per-token step runs n times).  Writes the KV
  * rows, leaves the last position's logits (cw_model_logits) and final-normed
  * hidden state (cw_model_hidden), returns its argmax in *next_token, and sets
  * the decode state to (next_token, start_pos + n). */

@@ -369,6 +369,58 @@ def test_prefill_qwen3_8b_layers_512(ctx):
     o.close()
 
 
+@pytest.mark.parametrize("kv", [cw.CW_F16, cw.CW_F32])
+@pytest.mark.parametrize("n_heads,n_kv", [(4, 4), (4, 2), (8, 2), (8, 1)])
+def test_prefill_attention_chunks(ctx, kv, n_heads, n_kv):
+    """The prompt phase behind a filled cache, at the edges of attention's
+    query tiles (16 positions a wave) and key tiles (64 keys, 32 for f32) and
+    with its keys in many chunks: logits within 1e-3 of the oracle's per-token
+    forward over the same cache."""
+    cfg = cw.make_config(1, 256, n_heads, n_kv, 128, 512, 500, 460, kv, 1e-6, 1e6)
+    weights = cw.synthetic_weights(cfg, 84 + n_heads + n_kv)
+    m = cw.Model(ctx, cfg)
+    m.set_weights(weights)
+    m.finalize()
+    es = np.float16 if kv == cw.CW_F16 else np.float32
+    rng = np.random.default_rng(84)
+    for start, P in ((0, 2), (0, 33), (0, 129), (31, 16), (63, 17), (64, 65), (333, 3),
+                     (389, 70)):
+        k, v = (rng.standard_normal((1, max(start, 1), n_kv * 128)).astype(es) for _ in range(2))
+        prompt = cw.synth_tokens(cw.synth_key(84, f"a{start}x{P}"), P, cfg.vocab)
+        o = orc.OracleModel(cfg, weights)
+        if start:
+            bits = np.uint16 if kv == cw.CW_F16 else np.float32
+            m.prefill_kv(k.view(bits), v.view(bits), start)
+            o.prefill_kv(k.view(bits), v.view(bits), start)
+        nxt = m.prefill(prompt, start_pos=start)
+        ref = oracle_prompt_logits(o, prompt, start)
+        diff = float(np.max(np.abs(m.logits() - ref)))
+        assert diff <= LOGIT_TOL, (start, P, diff)
+        assert nxt == int(np.argmax(ref)), (start, P)
+        o.close()
+    m.close()
+
+
+def test_prefill_rows_past_the_prompt_do_not_reach_it(ctx):
+    """Stale rows behind the prompt (NaN) leave the logits' bits unchanged."""
+    for kv, es in ((cw.CW_F16, np.float16), (cw.CW_F32, np.float32)):
+        cfg = cw.make_config(1, 256, 4, 2, 128, 512, 500, 256, kv, 1e-6, 1e6)
+        weights = cw.synthetic_weights(cfg, 85)
+        prompt = cw.synth_tokens(cw.synth_key(85, "p"), 37, cfg.vocab)
+        out = []
+        for fill in (0.0, np.nan):
+            m = cw.Model(ctx, cfg)
+            m.set_weights(weights)
+            m.finalize()
+            rows = np.full((1, 256, 256), fill, es)
+            bits = rows.view(np.uint16) if es is np.float16 else rows
+            m.prefill_kv(bits, bits, 256)
+            m.prefill(prompt)
+            out.append(m.logits())
+            m.close()
+        assert np.array_equal(out[0], out[1])
+
+
 def test_prefill_f32_cache_runs_per_token(ctx):
     """An f32 cache takes the per-token step for the prompt: same logits as
     the oracle's loop."""
