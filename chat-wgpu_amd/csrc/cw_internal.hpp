@@ -153,28 +153,29 @@ struct same_type {
     using type = T;
 };
 
-__device__ __forceinline__ float add(float a, float b) { return a + b; }
+__device__ __forceinline__ float2 add(float2 a, float2 b) {
+    return make_float2(a.x + b.x, a.y + b.y);
+}
 __device__ __forceinline__ float4 add(float4 a, float4 b) {
     return make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w);
 }
 
-// The sum in order of the S >= 1 partials at p, p + stride, ...: four
-// requested at a time, so that no load waits for another's sum.
-template <typename T>
-__device__ __forceinline__ T sum_parts(const float *p, int S, size_t stride) {
-    auto at = [&](int s) { return *reinterpret_cast<const T *>(p + (size_t)s * stride); };
-    T v = at(0);
+// The sum in order of the S >= 1 partials at(0), at(1), ...: four requested
+// at a time, so that no load waits for another's sum.
+template <typename At>
+__device__ __forceinline__ auto sum_parts(int S, At at) {
+    auto v = at(0);
     int s = 1;
     for (; s + 4 <= S; s += 4) {
-        const T a = at(s), b = at(s + 1), c = at(s + 2), d = at(s + 3);
+        const auto a = at(s), b = at(s + 1), c = at(s + 2), d = at(s + 3);
         v = add(add(add(add(v, a), b), c), d);
     }
     if (s + 3 == S) {
-        const T a = at(s), b = at(s + 1), c = at(s + 2);
+        const auto a = at(s), b = at(s + 1), c = at(s + 2);
         return add(add(add(v, a), b), c);
     }
     if (s + 2 == S) {
-        const T a = at(s), b = at(s + 1);
+        const auto a = at(s), b = at(s + 1);
         return add(add(v, a), b);
     }
     return s < S ? add(v, at(s)) : v;
@@ -312,7 +313,8 @@ int launch_argmax(cw_ctx *ctx, const float *logits, int n, uint32_t *out_dev, vo
 // silu(A x) * (B x).
 struct GemmArgs {
     const uint16_t *img;        // x image, gemm_img_elems(M, K) elements
-    const float *rowscale;      // [M] powers of two
+    const float *rowscale;      // [M] powers of two, or one set per K split:
+    int seg_blocks;             // blocks that share one (0: all), as the plan splits K
     const uint16_t *sA;
     const uint8_t *qA;
     const uint16_t *sB;
@@ -351,9 +353,13 @@ int launch_q4_gemm(cw_ctx *ctx, Epi epi, GemmArgs a, int *splits);
 int launch_gemm_reduce(cw_ctx *ctx, const GemmArgs &a, int splits);
 // The GEMM's result (its partials summed in the same pass) as the next GEMM's
 // split image, RMS-normalised with norm_w when set; y holds it too, but for
-// SwiGLU partials.
+// SwiGLU partials.  seg_blocks (SwiGLU partials only): row scales per that many
+// blocks, the K splits of the GEMM that follows.
 int launch_reduce_split(cw_ctx *ctx, Epi epi, const GemmArgs &a, int splits, const float *norm_w,
-                        float eps, uint16_t *img, float *rowscale);
+                        float eps, int seg_blocks, uint16_t *img, float *rowscale);
+// Blocks per K split of the GEMM's plan (as launch_q4_gemm will take it).
+int gemm_seg_blocks(const cw_ctx *ctx, Epi epi, int M, int N, int K, size_t part_floats);
+constexpr int kMaxSplits = 16;  // row scale sets at most
 // qkv: [M][q | k | v] rows, or (splits > 0) the sum in order of `splits`
 // partials part[s][M][q | k | v] (gemm_reduce_kernel's sum)
 int launch_qk_rope_kv(cw_ctx *ctx, const float *qkv, const float *qn, const float *kn, float eps,
@@ -382,9 +388,10 @@ AttnPrefillPlan attn_prefill_plan(const cw_ctx *ctx, int kv_dtype, int M, int n_
 // rows the plan of any prompt of up to M positions takes
 size_t attn_prefill_rows(const cw_ctx *ctx, int M, int n_heads, int n_kv);
 int launch_attn_prefill(cw_ctx *ctx, const AttnPrefillPlan &p, AttnPrefillArgs a, int kv_dtype);
-// The rows' split image for the O projection: of a.out, or of the merged chunks.
+// The rows' split image for the O projection: of a.out, or of the merged chunks
+// (row scales per seg_blocks blocks).
 int launch_attn_split(cw_ctx *ctx, const AttnPrefillPlan &p, const AttnPrefillArgs &a,
-                      uint16_t *img, float *rowscale);
+                      int seg_blocks, uint16_t *img, float *rowscale);
 
 // ---- the fused decode step (one persistent cooperative kernel per token)
 

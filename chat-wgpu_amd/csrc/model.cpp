@@ -509,7 +509,7 @@ int ensure_prefill(cw_model *m, int n) {
     CW_TRY(al((size_t)n * m->q_dim * 4, (void **)&m->pf_attn));
     CW_TRY(al((size_t)n * c.hidden * 4, (void **)&m->pf_act));
     CW_TRY(al(gemm_img_elems(n, (int)wide) * 2, (void **)&m->pf_img));
-    CW_TRY(al((size_t)n * 4, (void **)&m->pf_rowscale));
+    CW_TRY(al((size_t)n * kMaxSplits * 4, (void **)&m->pf_rowscale));
     // split-K partials of the largest plan (for n and for shorter prompts,
     // whose plans split further), and room for padded scales
     struct Shape {
@@ -540,11 +540,13 @@ int ensure_prefill(cw_model *m, int n) {
 }
 
 // The batched GEMM of one linear layer: y[n][out] = [resid +] x . W^T (SwiGLU
-// of two matrices), x being the split image in pf_img.  *splits as
+// of two matrices), x being the split image in pf_img (with row scales per
+// seg_blocks blocks, when set).  *splits as
 // launch_q4_gemm leaves it; the arguments come back for the pass that follows.
 int pf_gemm(cw_model *m, int n, int K, Epi epi, const Q4W &w, const Q4W *w2, const float *resid,
-            float *y, GemmArgs *out, int *splits) {
+            float *y, GemmArgs *out, int *splits, int seg_blocks = 0) {
     GemmArgs a{};
+    a.seg_blocks = seg_blocks;
     a.img = m->pf_img;
     a.rowscale = m->pf_rowscale;
     a.sA = w.s;
@@ -581,9 +583,13 @@ int enqueue_prefill(cw_model *m, int n, int start) {
     const auto &c = m->cfg;
     const float eps = c.eps;
     // a GEMM's result as the next one's operand, in one pass
-    auto to_image = [&](Epi epi, const GemmArgs &a, int splits, const float *norm_w) {
-        return launch_reduce_split(ctx, epi, a, splits, norm_w, eps, m->pf_img, m->pf_rowscale);
+    auto to_image = [&](Epi epi, const GemmArgs &a, int splits, const float *norm_w, int seg) {
+        return launch_reduce_split(ctx, epi, a, splits, norm_w, eps, seg, m->pf_img,
+                                   m->pf_rowscale);
     };
+    // the K splits of the O and down GEMMs, for their operands' row scales
+    const int seg_o = gemm_seg_blocks(ctx, EPI_ADD, n, c.dim, m->q_dim, m->pf_part_floats);
+    const int seg_d = gemm_seg_blocks(ctx, EPI_ADD, n, c.dim, c.hidden, m->pf_part_floats);
     GemmArgs g{};
     int splits = 0;
     CW_TRY(launch_embed_split(ctx, m->embed, m->prompt_dev, m->layers[0].attn_norm, eps, n, c.dim,
@@ -614,17 +620,19 @@ int enqueue_prefill(cw_model *m, int n, int start) {
         at.kc = kc;
         at.vc = vc;
         CW_TRY(launch_attn_prefill(ctx, plan, at, c.kv_dtype));
-        CW_TRY(launch_attn_split(ctx, plan, at, m->pf_img, m->pf_rowscale));
+        const int seg_a = plan.chunks > 1 ? seg_o : 0;
+        CW_TRY(launch_attn_split(ctx, plan, at, seg_a, m->pf_img, m->pf_rowscale));
         CW_TRY(pf_gemm(m, n, m->q_dim, EPI_ADD, L.wo, nullptr, m->pf_hidden, m->pf_hidden, &g,
-                       &splits));
-        CW_TRY(to_image(EPI_ADD, g, splits, L.ffn_norm));
+                       &splits, seg_a));
+        CW_TRY(to_image(EPI_ADD, g, splits, L.ffn_norm, 0));
         CW_TRY(tap_row(m, m->tap_post + (size_t)i * c.dim, m->pf_hidden, n - 1, c.dim));
         CW_TRY(pf_gemm(m, n, c.dim, EPI_SWIGLU, L.gate, &L.up, nullptr, m->pf_act, &g, &splits));
-        CW_TRY(to_image(EPI_SWIGLU, g, splits, nullptr));
+        const int seg_h = splits ? seg_d : 0;
+        CW_TRY(to_image(EPI_SWIGLU, g, splits, nullptr, seg_h));
         CW_TRY(pf_gemm(m, n, c.hidden, EPI_ADD, L.down, nullptr, m->pf_hidden, m->pf_hidden, &g,
-                       &splits));
+                       &splits, seg_h));
         if (i + 1 < c.n_layers)
-            CW_TRY(to_image(EPI_ADD, g, splits, m->layers[i + 1].attn_norm));
+            CW_TRY(to_image(EPI_ADD, g, splits, m->layers[i + 1].attn_norm, 0));
         else if (splits)
             CW_TRY(launch_gemm_reduce(ctx, g, splits));
         CW_TRY(tap_row(m, m->tap_out + (size_t)i * c.dim, m->pf_hidden, n - 1, c.dim));

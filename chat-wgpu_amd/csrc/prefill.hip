@@ -53,15 +53,21 @@ __global__ __launch_bounds__(kT) void qk_rope_kv_kernel(const float *__restrict_
     const int q_dim = n_heads * HD, kv_dim = n_kv * HD;
     const size_t row_off = (size_t)i * (q_dim + 2 * kv_dim);
     const float *row = (S > 0 ? part : qkv) + row_off;
-    // p: an element of row (of partial 0)
-    auto val = [&](const float *p) { return S > 0 ? cwi::sum_parts<float>(p, S, MN) : *p; };
+    // elements p[lane] and p[lane + 64] of row (of partial 0)
+    auto val = [&](const float *p) {
+        return cwi::sum_parts(max(S, 1), [&](int s2) {
+            const float *q = p + (size_t)s2 * MN + lane;
+            return make_float2(q[0], q[HALF]);
+        });
+    };
     const float c = cos_t[(size_t)pos * HALF + lane], s = sin_t[(size_t)pos * HALF + lane];
     // one head per wave: workgroup y takes heads 4 y .. 4 y + 3 of the row
     for (int h = blockIdx.y * (kT / 64) + wave; h < n_heads + n_kv; h += gridDim.y * (kT / 64)) {
         const bool isq = h < n_heads;
         const float *src = isq ? row + (size_t)h * HD : row + q_dim + (size_t)(h - n_heads) * HD;
         const float *g = isq ? qn : kn;
-        const float lo = val(src + lane), hi = val(src + lane + HALF);
+        const float2 x = val(src);
+        const float lo = x.x, hi = x.y;
         const float ss = wave_sum(lo * lo + hi * hi);
         const float inv = 1.0f / sqrtf(ss / (float)HD + eps);
         const float l0 = (lo * inv) * g[lane], h0 = (hi * inv) * g[lane + HALF];
@@ -77,8 +83,9 @@ __global__ __launch_bounds__(kT) void qk_rope_kv_kernel(const float *__restrict_
             kd[lane + HALF] = (KVT)r1;
             const float *vs = row + q_dim + kv_dim + (size_t)g2 * HD;
             KVT *vd = vc + (size_t)pos * kv_dim + (size_t)g2 * HD;
-            vd[lane] = (KVT)val(vs + lane);
-            vd[lane + HALF] = (KVT)val(vs + lane + HALF);
+            const float2 v = val(vs);
+            vd[lane] = (KVT)v.x;
+            vd[lane + HALF] = (KVT)v.y;
         }
     }
 }

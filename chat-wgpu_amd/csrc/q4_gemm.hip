@@ -51,8 +51,11 @@ constexpr float kUnscale = 0.0625f;  // the products' factor 16
 // the order in which the masks of a packed word yield the weights.
 // rowscale[row] = 2^e.
 //
-// One workgroup per row; a thread takes whole chunks (8 elements), CH of them
-// in registers.  Sources of a row: SRC_ROWS, x itself; SRC_PART, the sum in
+// One workgroup per row, or per (row, segment of the columns) with a row scale
+// for each: where the consumer splits K by the same segments, few long rows
+// still give every CU a workgroup (the SwiGLU pass of 24 rows of 12288: 15.6
+// us as 24 workgroups).  RMSNorm needs whole rows.  A thread takes whole
+// chunks (8 elements), CH of them in registers.  Sources of a row: SRC_ROWS, x itself; SRC_PART, the sum in
 // order of S split-K partials (+ resid), also written to y; SRC_SWIGLU,
 // silu(g) u of the summed partials of the gate and the up product; SRC_EMBED,
 // a token's embedding row (Qwen3::embed, qwen3.rs:128-133), also written to y;
@@ -73,9 +76,16 @@ struct SplitArgs {
     const float *norm_w;  // NORM: gain [K]
     float eps;
     int K;
+    int seg;  // chunks per segment
     uint16_t *img;
     float *rowscale;
 };
+
+__device__ __forceinline__ float4 sum4(const float *p, int S, size_t stride) {
+    return cwi::sum_parts(S, [&](int s) {
+        return *reinterpret_cast<const float4 *>(p + (size_t)s * stride);
+    });
+}
 
 __device__ __forceinline__ float silu_mul(float g, float u) { return g / (1.0f + expf(-g)) * u; }
 
@@ -83,7 +93,8 @@ template <bool NORM, int SRC, int CH>
 __global__ __launch_bounds__(512) void split_image_kernel(SplitArgs a) {
     __shared__ float red[2][8];
     const int tid = threadIdx.x, nt = blockDim.x, lane = tid & 63, wave = tid >> 6;
-    const int nch = a.K >> 3;  // chunks of the row
+    // the segment's chunks [c0, nch)
+    const int c0 = blockIdx.y * a.seg, nch = min(a.K >> 3, c0 + a.seg);
     const size_t base = (size_t)blockIdx.x * a.K;
     // elements 4 g .. of the block and 16 + 4 g .. for chunk c
     auto load8 = [&](int c, float4 &ve, float4 &vf) {
@@ -96,8 +107,8 @@ __global__ __launch_bounds__(512) void split_image_kernel(SplitArgs a) {
             float4 v[2];
 #pragma unroll
             for (int k = 0; k < 2; ++k) {
-                const float4 g = cwi::sum_parts<float4>(a.x + o + 16 * k, a.S, 2 * a.MK);
-                const float4 u = cwi::sum_parts<float4>(a.x + a.MK + o + 16 * k, a.S, 2 * a.MK);
+                const float4 g = sum4(a.x + o + 16 * k, a.S, 2 * a.MK);
+                const float4 u = sum4(a.x + a.MK + o + 16 * k, a.S, 2 * a.MK);
                 v[k] = make_float4(silu_mul(g.x, u.x), silu_mul(g.y, u.y), silu_mul(g.z, u.z),
                                    silu_mul(g.w, u.w));
             }
@@ -111,8 +122,10 @@ __global__ __launch_bounds__(512) void split_image_kernel(SplitArgs a) {
             const float2 *ml = reinterpret_cast<const float2 *>(a.ml) + blockIdx.x * heads +
                                col / 128;
             float m = -INFINITY, l = 0.0f;
+#pragma unroll 4
             for (int i = 0; i < n; ++i) m = fmaxf(m, ml[i * step].x);
             ve = vf = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll 4
             for (int i = 0; i < n; ++i) {
                 const float2 p = ml[i * step];
                 const float f = __builtin_amdgcn_exp2f(p.x - m);
@@ -135,7 +148,7 @@ __global__ __launch_bounds__(512) void split_image_kernel(SplitArgs a) {
             float4 v[2];
 #pragma unroll
             for (int k = 0; k < 2; ++k) {
-                v[k] = cwi::sum_parts<float4>(a.x + o + 16 * k, a.S, a.MK);
+                v[k] = sum4(a.x + o + 16 * k, a.S, a.MK);
                 if (a.resid) {
                     const float4 r = *reinterpret_cast<const float4 *>(a.resid + o + 16 * k);
                     v[k] = make_float4(r.x + v[k].x, r.y + v[k].y, r.z + v[k].z, r.w + v[k].w);
@@ -173,11 +186,11 @@ __global__ __launch_bounds__(512) void split_image_kernel(SplitArgs a) {
     // is read again for the second pass
     float4 ve[CH], vf[CH];
 #pragma unroll
-    for (int j = 0; j < CH; ++j) load8(min(tid + j * nt, nch - 1), ve[j], vf[j]);
+    for (int j = 0; j < CH; ++j) load8(min(c0 + tid + j * nt, nch - 1), ve[j], vf[j]);
 #pragma unroll
     for (int j = 0; j < CH; ++j)
-        if (tid + j * nt < nch) scan(tid + j * nt, ve[j], vf[j]);
-    for (int c = tid + CH * nt; c < nch; c += nt) {
+        if (c0 + tid + j * nt < nch) scan(c0 + tid + j * nt, ve[j], vf[j]);
+    for (int c = c0 + tid + CH * nt; c < nch; c += nt) {
         float4 e, f;
         load8(c, e, f);
         scan(c, e, f);
@@ -202,7 +215,7 @@ __global__ __launch_bounds__(512) void split_image_kernel(SplitArgs a) {
     mx *= inv;
     const int e = mx > 0.0f ? max(ilogbf(mx) - 10, -126) : 0;
     const float sc = ldexpf(1.0f, -e);
-    if (tid == 0) a.rowscale[blockIdx.x] = ldexpf(1.0f, e);
+    if (tid == 0) a.rowscale[blockIdx.y * gridDim.x + blockIdx.x] = ldexpf(1.0f, e);
     auto emit = [&](int c, float4 ve, float4 vf) {
         const int b = c >> 2, g = c & 3;
         float v[8] = {ve.x, ve.y, ve.z, ve.w, vf.x, vf.y, vf.z, vf.w};
@@ -222,7 +235,7 @@ __global__ __launch_bounds__(512) void split_image_kernel(SplitArgs a) {
             hb[k] = __builtin_bit_cast(uint16_t, h);
             lb[k] = __builtin_bit_cast(uint16_t, (_Float16)(t - (float)h));
         }
-        uint16_t *p = a.img + (((size_t)blockIdx.x * (nch >> 2) + b) << 6) + 8 * g;
+        uint16_t *p = a.img + (((size_t)blockIdx.x * (a.K >> 5) + b) << 6) + 8 * g;
         *reinterpret_cast<uint4 *>(p) = make_uint4(hb[0] | hb[2] << 16, hb[4] | hb[6] << 16,
                                                    hb[1] | hb[3] << 16, hb[5] | hb[7] << 16);
         *reinterpret_cast<uint4 *>(p + 32) = make_uint4(lb[0] | lb[2] << 16, lb[4] | lb[6] << 16,
@@ -230,8 +243,8 @@ __global__ __launch_bounds__(512) void split_image_kernel(SplitArgs a) {
     };
 #pragma unroll
     for (int j = 0; j < CH; ++j)
-        if (tid + j * nt < nch) emit(tid + j * nt, ve[j], vf[j]);
-    for (int c = tid + CH * nt; c < nch; c += nt) {
+        if (c0 + tid + j * nt < nch) emit(c0 + tid + j * nt, ve[j], vf[j]);
+    for (int c = c0 + tid + CH * nt; c < nch; c += nt) {
         float4 e, f;
         if constexpr (SRC == SRC_PART) {  // this thread's own stores
             const size_t o = base + (size_t)(c >> 2) * 32 + 4 * (c & 3);
@@ -252,7 +265,7 @@ __global__ __launch_bounds__(kT) void gemm_reduce_kernel(const float *__restrict
     const bool vec = n % 4 == 0 && ((reinterpret_cast<uintptr_t>(y) |
                                      reinterpret_cast<uintptr_t>(resid)) & 15) == 0;
     if (vec) {
-        float4 v = cwi::sum_parts<float4>(part + i, S, n);
+        float4 v = sum4(part + i, S, n);
         if (resid) {
             const float4 r = *reinterpret_cast<const float4 *>(resid + i);
             v.x = r.x + v.x;
@@ -576,13 +589,14 @@ void q4_gemm_kernel(cwi::GemmArgs a, int MT, int NT, int S, int per) {
         for (int r = 0; r < 4; ++r)
             acc[i][CT - 1][r] = __builtin_fmaf(dp, t[1][i][r], acc[i][CT - 1][r]);
 
+    const float *const rsp = a.rowscale + (a.seg_blocks ? (size_t)sp * a.M : 0);
     constexpr int JN = SWI ? (CT + 1) / 2 : CT;
 #pragma unroll
     for (int i = 0; i < RT; ++i)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const int m = m0 + (wm * RT + i) * 16 + 4 * lg + r;
-            const float rs = a.rowscale[min(m, a.M - 1)];
+            const float rs = rsp[min(m, a.M - 1)];
 #pragma unroll
             for (int j = 0; j < JN; ++j) {
                 int n = n0 + (wn * JN + j) * 16 + li;
@@ -666,7 +680,7 @@ GemmPlan gemm_plan(const cw_ctx *ctx, cwi::Epi epi, int M, int N, int K, size_t 
         const Tile &T = kTiles[t];
         if (T.bm < kRowPad && M > 2 * T.bm) continue;
         const int MT = (M + T.bm - 1) / T.bm, NT = (cols + T.bn - 1) / T.bn;
-        for (int S : {1, 2, 3, 4, 6, 8, 12, 16}) {
+        for (int S : {1, 2, 3, 4, 6, 8, 12, cwi::kMaxSplits}) {
             const int per = ((nb + S - 1) / S + 7) / 8 * 8;  // whole scale groups
             if (S > 1 && ((nb + per - 1) / per != S ||
                           (size_t)S * M * cols > part_floats))
@@ -706,14 +720,15 @@ bool scales_in_groups(int K, const void *s) {
 }
 
 template <bool NORM, int SRC>
-int launch_split_image(cw_ctx *ctx, const char *label, const SplitArgs &a, int rows) {
-    // whole waves, no more than the row has chunks for; rows of up to 12,288
-    // stay in registers between the two passes
-    const int nch = a.K / 8, nt = std::min(512, (nch + 63) / 64 * 64);
-    if (nch <= nt)
-        return cwi::launch(ctx, label, split_image_kernel<NORM, SRC, 1>, dim3(rows), dim3(nt), 0,
-                           a);
-    return cwi::launch(ctx, label, split_image_kernel<NORM, SRC, 3>, dim3(rows), dim3(nt), 0, a);
+int launch_split_image(cw_ctx *ctx, const char *label, SplitArgs a, int rows, int seg_blocks = 0) {
+    // whole waves, no more than the row (segment) has chunks for; up to 12,288
+    // elements stay in registers between the two passes
+    a.seg = seg_blocks ? seg_blocks * 4 : a.K / 8;
+    const int nt = std::min(512, (a.seg + 63) / 64 * 64);
+    const dim3 grid(rows, (a.K / 8 + a.seg - 1) / a.seg);
+    if (a.seg <= nt)
+        return cwi::launch(ctx, label, split_image_kernel<NORM, SRC, 1>, grid, dim3(nt), 0, a);
+    return cwi::launch(ctx, label, split_image_kernel<NORM, SRC, 3>, grid, dim3(nt), 0, a);
 }
 
 }  // namespace
@@ -731,6 +746,10 @@ size_t gemm_spad_elems(int N, int K, const void *scales) {
 size_t gemm_part_floats(const cw_ctx *ctx, Epi epi, int M, int N, int K) {
     const GemmPlan p = gemm_plan(ctx, epi, M, N, K, SIZE_MAX);
     return p.S > 1 ? (size_t)p.S * M * w_cols(epi, N) : 0;
+}
+
+int gemm_seg_blocks(const cw_ctx *ctx, Epi epi, int M, int N, int K, size_t part_floats) {
+    return gemm_plan(ctx, epi, M, N, K, part_floats).per;
 }
 
 int launch_split_rows(cw_ctx *ctx, const float *x, const float *norm_w, float eps, int rows, int K,
@@ -762,7 +781,7 @@ int launch_embed_split(cw_ctx *ctx, const float *table, const uint32_t *tok_dev,
 }
 
 int launch_attn_split(cw_ctx *ctx, const AttnPrefillPlan &p, const AttnPrefillArgs &t,
-                      uint16_t *img, float *rowscale) {
+                      int seg_blocks, uint16_t *img, float *rowscale) {
     const int K = t.n_heads * 128;
     if (p.chunks == 1) return launch_split_rows(ctx, t.out, nullptr, 0.0f, t.M, K, img, rowscale);
     SplitArgs a{};
@@ -776,7 +795,8 @@ int launch_attn_split(cw_ctx *ctx, const AttnPrefillPlan &p, const AttnPrefillAr
     a.K = K;
     a.img = img;
     a.rowscale = rowscale;
-    return launch_split_image<false, SRC_ATTN>(ctx, "prefill_attention_merge", a, t.M);
+    return launch_split_image<false, SRC_ATTN>(ctx, "prefill_attention_merge", a, t.M,
+                                               seg_blocks);
 }
 
 int launch_q4_gemm(cw_ctx *ctx, Epi epi, GemmArgs a, int *splits) {
@@ -816,7 +836,7 @@ int launch_gemm_reduce(cw_ctx *ctx, const GemmArgs &a, int splits) {
 }
 
 int launch_reduce_split(cw_ctx *ctx, Epi epi, const GemmArgs &g, int splits, const float *norm_w,
-                        float eps, uint16_t *img, float *rowscale) {
+                        float eps, int seg_blocks, uint16_t *img, float *rowscale) {
     SplitArgs a{};
     a.x = splits ? g.part : g.y;
     a.S = splits;
@@ -830,7 +850,8 @@ int launch_reduce_split(cw_ctx *ctx, Epi epi, const GemmArgs &g, int splits, con
     a.rowscale = rowscale;
     if (!splits) return launch_split_rows(ctx, g.y, norm_w, eps, g.M, g.N, img, rowscale);
     if (epi == EPI_SWIGLU)
-        return launch_split_image<false, SRC_SWIGLU>(ctx, "q4_gemm_reduce_swiglu", a, g.M);
+        return launch_split_image<false, SRC_SWIGLU>(ctx, "q4_gemm_reduce_swiglu", a, g.M,
+                                                     seg_blocks);
     return norm_w ? launch_split_image<true, SRC_PART>(ctx, "q4_gemm_reduce_split", a, g.M)
                   : launch_split_image<false, SRC_PART>(ctx, "q4_gemm_reduce_split", a, g.M);
 }
