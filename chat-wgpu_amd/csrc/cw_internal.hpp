@@ -296,6 +296,7 @@ struct GenState {
     int produced;
     int max_out;
 };
+int launch_set_state(cw_ctx *ctx, const GenState &s, GenState *dst);
 size_t argmax_scratch_bytes(int n);
 // Scratch of the LM head's fused argmax (EPI_ARGMAX): per-workgroup bests
 // for any grid launch_q4_gemv picks, then the arrival counter line.

@@ -70,6 +70,10 @@ struct cw_model {
     float *part = nullptr;
     void *argmax_scratch = nullptr;
     void *lm_scratch = nullptr;  // the LM head's fused argmax (counter zero between launches)
+    // pinned host memory: max_seq token ids on their way to prompt_dev, then
+    // the last argmax; `stage_busy` while a copy may still read the ids
+    uint32_t *stage = nullptr;
+    bool stage_busy = false;
     int host_pos = 0;            // the device state's pos, mirrored (every step advances it by 1)
     GenState *state = nullptr;
     uint32_t *prompt_dev = nullptr, *tokens_dev = nullptr, *argmax_out = nullptr;
@@ -328,7 +332,7 @@ int ensure_graph(cw_model *m) {
 // The fused step's counters after a launch sequence: a set error word means
 // a grid barrier timed out; the counters are cleared for the next launch.
 int check_fused(cw_model *m) {
-    if (!m->step_sync) return CW_OK;
+    if (!m->step_sync || kFusedStepDisabled) return CW_OK;  // (no launch can have set it)
     unsigned err = 0;
     CW_HIP(hipMemcpyAsync(&err, m->step_sync + step_sync_err_index(), 4, hipMemcpyDeviceToHost,
                           m->ctx->stream));
@@ -486,16 +490,16 @@ int setup_fused(cw_model *m) {
     return CW_OK;
 }
 
-// Batched prefill buffers for n positions.
-int ensure_prefill(cw_model *m, int n) {
-    if (n <= m->pf_cap) return CW_OK;
-    CW_HIP(hipStreamSynchronize(m->ctx->stream));
-    for (void *p : m->pf_allocs) CW_HIP(hipFree(p));
+void free_prefill(cw_model *m) {
+    for (void *p : m->pf_allocs) (void)hipFree(p);
     m->pf_allocs.clear();
     m->pf_cap = 0;
     m->pf_part = nullptr;
     m->pf_part_floats = 0;
     m->pf_spad = nullptr;
+}
+
+int alloc_prefill(cw_model *m, int n) {
     const auto &c = m->cfg;
     const size_t wide = std::max({(size_t)c.dim, (size_t)m->q_dim, (size_t)c.hidden});
     auto al = [&](size_t bytes, void **out) -> int {
@@ -539,6 +543,17 @@ int ensure_prefill(cw_model *m, int n) {
     return CW_OK;
 }
 
+// Batched prefill buffers for n positions; none are left behind when there is
+// no room for all of them.
+int ensure_prefill(cw_model *m, int n) {
+    if (n <= m->pf_cap) return CW_OK;
+    CW_HIP(hipStreamSynchronize(m->ctx->stream));
+    free_prefill(m);
+    const int rc = alloc_prefill(m, n);
+    if (rc != CW_OK) free_prefill(m);
+    return rc;
+}
+
 // The batched GEMM of one linear layer: y[n][out] = [resid +] x . W^T (SwiGLU
 // of two matrices), x being the split image in pf_img (with row scales per
 // seg_blocks blocks, when set).  *splits as
@@ -575,10 +590,10 @@ int tap_row(cw_model *m, float *dst, const float *src, int row, int floats) {
     return CW_OK;
 }
 
-// Forward of n positions start..start+n-1 (tokens in m->prompt_dev) through
+// Forward of n positions start..start+n-1 (tokens in prompt_dev from `tok`) through
 // every layer with the batched kernels; leaves the hidden rows in pf_hidden.
 // With taps on, the taps are those of the last position's forward.
-int enqueue_prefill(cw_model *m, int n, int start) {
+int enqueue_prefill(cw_model *m, int tok, int n, int start) {
     cw_ctx *ctx = m->ctx;
     const auto &c = m->cfg;
     const float eps = c.eps;
@@ -592,7 +607,7 @@ int enqueue_prefill(cw_model *m, int n, int start) {
     const int seg_d = gemm_seg_blocks(ctx, EPI_ADD, n, c.dim, c.hidden, m->pf_part_floats);
     GemmArgs g{};
     int splits = 0;
-    CW_TRY(launch_embed_split(ctx, m->embed, m->prompt_dev, m->layers[0].attn_norm, eps, n, c.dim,
+    CW_TRY(launch_embed_split(ctx, m->embed, m->prompt_dev + tok, m->layers[0].attn_norm, eps, n, c.dim,
                               m->pf_hidden, m->pf_img, m->pf_rowscale));
     const AttnPrefillPlan plan = attn_prefill_plan(ctx, c.kv_dtype, n, c.n_heads, c.n_kv_heads,
                                                    start, m->pf_attn_rows);
@@ -641,11 +656,63 @@ int enqueue_prefill(cw_model *m, int n, int start) {
 }
 
 int set_state(cw_model *m, const GenState &s) {
-    CW_HIP(hipMemcpyAsync(m->state, &s, sizeof s, hipMemcpyHostToDevice, m->ctx->stream));
-    CW_HIP(hipStreamSynchronize(m->ctx->stream));
+    CW_TRY(launch_set_state(m->ctx, s, m->state));
     m->host_pos = s.pos;
     return CW_OK;
 }
+
+// Token ids to prompt_dev through pinned memory, without waiting for the copy.
+int stage_prompt(cw_model *m, const uint32_t *tokens, int n) {
+    if (m->stage_busy) CW_HIP(hipStreamSynchronize(m->ctx->stream));
+    memcpy(m->stage, tokens, (size_t)n * 4);
+    m->stage_busy = true;
+    CW_HIP(hipMemcpyAsync(m->prompt_dev, m->stage, (size_t)n * 4, hipMemcpyHostToDevice,
+                          m->ctx->stream));
+    return CW_OK;
+}
+
+// The last argmax, once the stream has drained.
+int read_argmax(cw_model *m, uint32_t *out) {
+    uint32_t *r = m->stage + m->cfg.max_seq;
+    CW_HIP(hipMemcpyAsync(r, m->argmax_out, 4, hipMemcpyDeviceToHost, m->ctx->stream));
+    CW_HIP(hipStreamSynchronize(m->ctx->stream));
+    m->stage_busy = false;
+    *out = *r;
+    return CW_OK;
+}
+
+// The batched prompt phase of the n tokens in prompt_dev: every position
+// through every layer, kPrefillChunk at a time (the buffers hold one chunk),
+// then the last position's logits and argmax, advancing the decode state when
+// given.  *last: its hidden row.
+constexpr int kPrefillChunk = 4096;
+int run_prefill(cw_model *m, int n, int start, GenState *state, const float **last) {
+    const auto &c = m->cfg;
+    CW_TRY(ensure_prefill(m, std::min(n, kPrefillChunk)));
+    int rows = 0;
+    for (int i = 0; i < n; i += rows) {
+        rows = std::min(n - i, kPrefillChunk);
+        CW_TRY(enqueue_prefill(m, i, rows, start + i));
+    }
+    *last = m->pf_hidden + (size_t)(rows - 1) * c.dim;
+    GemvArgs g{};
+    g.x = *last;
+    g.norm_w = m->final_norm;
+    g.eps = c.eps;
+    g.sA = m->lm_head.s;
+    g.qA = m->lm_head.q;
+    g.y = m->logits;
+    g.K = c.dim;
+    g.N = c.vocab;
+    return launch_lm_head_argmax(m->ctx, g, m->lm_scratch, m->argmax_out, state, m->prompt_dev,
+                                 m->tokens_dev);
+}
+
+// Prompts that go through run_prefill: head_dim 128 (what its attention is
+// built for) and more than one position (two 8B layers: 118 us for one token
+// by a step, 205 for two, 293 for three; 192 for a batch of 2 to 8; four 0.6B
+// layers: 133, 249 and 358 against 210).
+bool batched_prompt(const cw_model *m, int n) { return m->cfg.head_dim == 128 && n > 1; }
 
 int require_final(cw_model *m, const char *what) {
     if (!m->finalized) {
@@ -769,6 +836,12 @@ int cw_model_create(cw_ctx *ctx, const cw_model_config *cfg, cw_model **out) {
     cw_model *m = new cw_model();
     m->ctx = ctx;
     int rc = model_alloc(m, c);
+    if (rc == CW_OK &&
+        hipHostMalloc((void **)&m->stage, (size_t)(c.max_seq + 1) * 4, hipHostMallocDefault) !=
+            hipSuccess) {
+        set_error("cw_model_create: %d bytes of pinned host memory", (c.max_seq + 1) * 4);
+        rc = CW_ERR_OOM;
+    }
     if (rc != CW_OK) {
         cw_model_destroy(m);
         return rc;
@@ -853,7 +926,8 @@ int cw_model_destroy(cw_model *m) {
     if (m->graph_exec) (void)hipGraphExecDestroy(m->graph_exec);
     if (m->graph) (void)hipGraphDestroy(m->graph);
     for (void *p : m->allocs) (void)hipFree(p);
-    for (void *p : m->pf_allocs) (void)hipFree(p);
+    free_prefill(m);
+    if (m->stage) (void)hipHostFree(m->stage);
     delete m;
     return CW_OK;
 }
@@ -1066,8 +1140,7 @@ int cw_model_step(cw_model *m, uint32_t token, int pos, uint32_t *argmax_out) {
     CW_TRY(launch_rmsnorm(m->ctx, last_hidden(m), m->final_norm, 1, m->cfg.dim, m->cfg.eps,
                           m->hidden_out));
     uint32_t r = 0;
-    CW_HIP(hipMemcpyAsync(&r, m->argmax_out, 4, hipMemcpyDeviceToHost, m->ctx->stream));
-    CW_HIP(hipStreamSynchronize(m->ctx->stream));
+    CW_TRY(read_argmax(m, &r));
     if (argmax_out) *argmax_out = r;
     return CW_OK;
 }
@@ -1154,13 +1227,32 @@ int cw_generate(cw_model *m, const uint32_t *prompt, int n_prompt, int max_new, 
     for (int i = 0; i < n_prompt; ++i)
         CW_CHECK_ARG(prompt[i] < (uint32_t)m->cfg.vocab, "cw_generate: prompt[%d]=%u >= vocab", i,
                      prompt[i]);
-    CW_TRY(cw_upload(m->ctx, m->prompt_dev, prompt, (size_t)n_prompt * 4));
-    GenState s{start_pos, prompt[0], start_pos, n_prompt, 0, max_new};
-    CW_TRY(set_state(m, s));
-    CW_TRY(run_steps(m, (int)total, mode));
+    CW_TRY(stage_prompt(m, prompt, n_prompt));
+    int steps = (int)total;
+    bool batched = mode == CW_STEP_GRAPH && batched_prompt(m, n_prompt);
+    if (batched) {
+        // the prompt's forwards at once; the LM head then advances the state
+        // as the last of them would
+        const int rc = ensure_prefill(m, std::min(n_prompt, kPrefillChunk));
+        batched = rc == CW_OK;
+        if (rc != CW_OK && rc != CW_ERR_OOM) return rc;
+        if (!batched) (void)hipGetLastError();  // no room for its buffers: step by step
+    }
+    if (batched) {
+        const int at = start_pos + n_prompt - 1;
+        CW_TRY(set_state(m, GenState{at, prompt[n_prompt - 1], start_pos, n_prompt, 0, max_new}));
+        const float *last = nullptr;
+        CW_TRY(run_prefill(m, n_prompt, start_pos, m->state, &last));
+        m->host_pos = at + 1;
+        steps = max_new - 1;
+    } else {
+        CW_TRY(set_state(m, GenState{start_pos, prompt[0], start_pos, n_prompt, 0, max_new}));
+    }
+    CW_TRY(run_steps(m, steps, mode));
     CW_HIP(hipMemcpyAsync(out_tokens, m->tokens_dev, (size_t)max_new * 4, hipMemcpyDeviceToHost,
                           m->ctx->stream));
     CW_HIP(hipStreamSynchronize(m->ctx->stream));
+    m->stage_busy = false;
     return check_fused(m);
 }
 
@@ -1176,38 +1268,19 @@ int cw_model_prefill(cw_model *m, const uint32_t *tokens, int n, int start_pos,
     for (int i = 0; i < n; ++i)
         CW_CHECK_ARG(tokens[i] < (uint32_t)c.vocab, "cw_model_prefill: tokens[%d]=%u >= vocab", i,
                      tokens[i]);
-    CW_TRY(cw_upload(m->ctx, m->prompt_dev, tokens, (size_t)n * 4));
-    // head_dim 128 (either cache type) and more than one position
-    const bool batched = c.head_dim == 128 && n > 1;
-    if (batched) {
-        CW_TRY(ensure_prefill(m, n));
-        CW_TRY(enqueue_prefill(m, n, start_pos));
-        // the last position's logits (the prompt phase discards the others,
-        // mod.rs:93-103) and the final-normed hidden state
-        const float *last = m->pf_hidden + (size_t)(n - 1) * c.dim;
-        GemvArgs g{};
-        g.x = last;
-        g.norm_w = m->final_norm;
-        g.eps = c.eps;
-        g.sA = m->lm_head.s;
-        g.qA = m->lm_head.q;
-        g.y = m->logits;
-        g.K = c.dim;
-        g.N = c.vocab;
-        CW_TRY(launch_lm_head_argmax(m->ctx, g, m->lm_scratch, m->argmax_out, nullptr, nullptr,
-                                     nullptr));
-        CW_TRY(launch_rmsnorm(m->ctx, last, m->final_norm, 1, c.dim, c.eps, m->hidden_out));
+    CW_TRY(stage_prompt(m, tokens, n));
+    const float *last = nullptr;
+    if (batched_prompt(m, n)) {
+        CW_TRY(run_prefill(m, n, start_pos, nullptr, &last));
     } else {
-        // another head_dim, or a single token: the per-token step, n times
-        GenState s{start_pos, tokens[0], start_pos, n, 0, 0};
-        CW_TRY(set_state(m, s));
+        CW_TRY(set_state(m, GenState{start_pos, tokens[0], start_pos, n, 0, 0}));
         CW_TRY(run_steps(m, n, CW_STEP_EAGER));
-        CW_TRY(launch_rmsnorm(m->ctx, last_hidden(m), m->final_norm, 1, c.dim, c.eps,
-                              m->hidden_out));
+        last = last_hidden(m);
     }
+    // the logits of all but the last position are discarded (mod.rs:93-103)
+    CW_TRY(launch_rmsnorm(m->ctx, last, m->final_norm, 1, c.dim, c.eps, m->hidden_out));
     uint32_t r = 0;
-    CW_HIP(hipMemcpyAsync(&r, m->argmax_out, 4, hipMemcpyDeviceToHost, m->ctx->stream));
-    CW_HIP(hipStreamSynchronize(m->ctx->stream));
+    CW_TRY(read_argmax(m, &r));
     if (next_token) *next_token = r;
     // decoding continues at start_pos + n with the predicted token
     GenState s{start_pos + n, r, start_pos + n, 1, 0, c.max_seq};
@@ -1242,8 +1315,7 @@ int cw_model_decode_next(cw_model *m, uint32_t *next_out) {
     CW_TRY(run_steps(m, 1, CW_STEP_GRAPH));
     // the step's LM head leaves its argmax here: one 4-byte read per token
     uint32_t r = 0;
-    CW_HIP(hipMemcpyAsync(&r, m->argmax_out, 4, hipMemcpyDeviceToHost, m->ctx->stream));
-    CW_HIP(hipStreamSynchronize(m->ctx->stream));
+    CW_TRY(read_argmax(m, &r));
     *next_out = r;
     return CW_OK;
 }

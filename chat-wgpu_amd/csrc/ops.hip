@@ -192,6 +192,10 @@ __global__ __launch_bounds__(kThreads) void argmax_final_kernel(const float *__r
     }
 }
 
+// The decode state from the launch's own argument: nothing on the host has to
+// outlive the call, so the caller need not wait for a copy.
+__global__ void set_state_kernel(cwi::GenState s, cwi::GenState *dst) { *dst = s; }
+
 // HBM read probe (the examples/q4probe.rs analogue): every thread streams
 // 16-byte words over a grid-stride loop and folds them with XOR, so nothing
 // but the reads costs time; one word per workgroup is written out.  The
@@ -273,6 +277,10 @@ int launch_embed(cw_ctx *ctx, const float *table, int vocab, int dim, const uint
     int blocks = (dim + kThreads - 1) / kThreads;
     return launch(ctx, "embed", embed_kernel, dim3(blocks), dim3(kThreads), 0, table, vocab, dim,
                   tok_dev, out);
+}
+
+int launch_set_state(cw_ctx *ctx, const GenState &s, GenState *dst) {
+    return launch(ctx, "set_state", set_state_kernel, dim3(1), dim3(1), 0, s, dst);
 }
 
 size_t argmax_scratch_bytes(int n) {

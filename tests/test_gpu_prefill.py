@@ -401,6 +401,31 @@ def test_prefill_attention_chunks(ctx, kv, n_heads, n_kv):
     m.close()
 
 
+@pytest.mark.parametrize("kv", [cw.CW_F16, cw.CW_F32])
+@pytest.mark.parametrize("P,start", [(1, 0), (3, 0), (4, 0), (37, 0), (5, 20)])
+def test_generate_batches_its_prompt(ctx, kv, P, start):
+    """generate's ids are the oracle's for prompts below and above the length
+    that goes through the batched prompt phase, alone and behind a cache, and
+    for a single new token; the state it leaves decodes on."""
+    cfg = cw.make_config(2, 256, 4, 2, 128, 512, 1000, 96, kv, 1e-6, 1e6)
+    weights = cw.synthetic_weights(cfg, 86)
+    prompt = cw.synth_tokens(cw.synth_key(86, f"p{P}"), P + start, cfg.vocab)
+    m = cw.Model(ctx, cfg)
+    m.set_weights(weights)
+    m.finalize()
+    o = orc.OracleModel(cfg, weights)
+    ref, _ = o.generate(prompt, 9)
+    for new in (1, 7):
+        if start:
+            m.prefill(prompt[:start])
+        toks = m.generate(prompt[start:], new, start_pos=start)
+        assert np.array_equal(toks, ref[:new]), (new, toks, ref)
+        assert np.array_equal(m.tokens(16), ref[:new])
+        assert m.decode_next() == int(ref[new])
+    m.close()
+    o.close()
+
+
 def test_prefill_rows_past_the_prompt_do_not_reach_it(ctx):
     """Stale rows behind the prompt (NaN) leave the logits' bits unchanged."""
     for kv, es in ((cw.CW_F16, np.float16), (cw.CW_F32, np.float32)):
