@@ -45,10 +45,13 @@ constexpr int kT = 256;
 constexpr float kUnscale = 0.0625f;  // the products' factor 16
 
 // ---------------------------------------------------------------------------
-// The x image: one 128-byte line per (row, block): 64 bytes of x_hi, then 64
-// of x_lo, each four 16-byte chunks g = 0..3 of the elements
-//   e0 e2 f0 f2 e1 e3 f1 f3   (e_i = 16 x[4 g + i], f_i = x[16 + 4 g + i]),
-// the order in which the masks of a packed word yield the weights.
+// The x image: per 16 rows and block 1 KB of x_hi, then 1 KB of x_lo, each as
+// the MFMA's lanes take it: lane 16 g + r has the 16-byte chunk
+//   e0 e2 f0 f2 e1 e3 f1 f3   (e_i = 16 x[4 g + i], f_i = x[16 + 4 g + i])
+// of row r, the order in which the masks of a packed word yield the weights.  So
+// a fragment is 1 KB of consecutive bytes, in memory as in LDS, and one DMA (as
+// 128 bytes per row and block, whose DMAs touch 16 places: 512 rows of 4096 ->
+// 6144 73.7 instead of 63.9 us).
 // rowscale[row] = 2^e.
 //
 // One workgroup per row, or per (row, segment of the columns) with a row scale
@@ -71,8 +74,9 @@ struct SplitArgs {
     float *y;             // SRC_PART, SRC_EMBED: [M][K]
     const uint32_t *tok;  // SRC_EMBED
     const float *ml;      // SRC_ATTN: (max log2 e, sum) [S][M][K / 128]
-    int M, start, pt, span;  // SRC_ATTN: rows, first position, positions that
-                             // share their chunks, positions per chunk
+    int start, pt, span;  // SRC_ATTN: first position, positions that share their
+                          // chunks, positions per chunk
+    int M;                // rows
     const float *norm_w;  // NORM: gain [K]
     float eps;
     int K;
@@ -89,18 +93,29 @@ __device__ __forceinline__ float4 sum4(const float *p, int S, size_t stride) {
 
 __device__ __forceinline__ float silu_mul(float g, float u) { return g / (1.0f + expf(-g)) * u; }
 
-template <bool NORM, int SRC, int CH>
-__global__ __launch_bounds__(512) void split_image_kernel(SplitArgs a) {
-    __shared__ float red[2][8];
-    const int tid = threadIdx.x, nt = blockDim.x, lane = tid & 63, wave = tid >> 6;
+// With R = 4 a workgroup takes four rows, neighbouring lanes the same chunk of
+// each, so a store covers 64 bytes of an image line instead of 16 (3000 rows of
+// 12288: 58 us; 80 with one row, 141 with one row and in plain row order).
+template <bool NORM, int SRC, int CH, int R>
+__global__ __launch_bounds__(R == 1 ? 512 : 1024) void split_image_kernel(SplitArgs a) {
+    __shared__ float red[2][R == 1 ? 8 : 16][R];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    // this thread's row of the workgroup's, and its place among that row's threads
+    const int ri = threadIdx.x % R, tid = threadIdx.x / R, nt = blockDim.x / R;
     // the segment's chunks [c0, nch)
     const int c0 = blockIdx.y * a.seg, nch = min(a.K >> 3, c0 + a.seg);
-    const size_t base = (size_t)blockIdx.x * a.K;
+    // workgroups go round-robin over the 8 XCDs: within 128 rows each XCD takes
+    // the 16 that share their image lines, which then meet in its L2
+    const int at = blockIdx.x * R, in = (at & 127) / R;
+    const int row0 = (at | 127) < a.M ? (at & ~127) + (in & 7) * 16 + (in >> 3) * R : at;
+    const bool mine = row0 + ri < a.M;  // (rows past the last read it again)
+    const int row = min(row0 + ri, a.M - 1);
+    const size_t base = (size_t)row * a.K;
     // elements 4 g .. of the block and 16 + 4 g .. for chunk c
     auto load8 = [&](int c, float4 &ve, float4 &vf) {
         const size_t col = (size_t)(c >> 2) * 32 + 4 * (c & 3), o = base + col;
         if constexpr (SRC == SRC_ROWS || SRC == SRC_EMBED) {
-            const float *p = a.x + (SRC == SRC_EMBED ? (size_t)a.tok[blockIdx.x] * a.K + col : o);
+            const float *p = a.x + (SRC == SRC_EMBED ? (size_t)a.tok[row] * a.K + col : o);
             ve = *reinterpret_cast<const float4 *>(p);
             vf = *reinterpret_cast<const float4 *>(p + 16);
         } else if constexpr (SRC == SRC_SWIGLU) {
@@ -116,10 +131,10 @@ __global__ __launch_bounds__(512) void split_image_kernel(SplitArgs a) {
             vf = v[1];
         } else if constexpr (SRC == SRC_ATTN) {
             // the chunks that reach the last key of this position's tile
-            const int last = a.start + min(((int)blockIdx.x / a.pt + 1) * a.pt, a.M) - 1;
+            const int last = a.start + min((row / a.pt + 1) * a.pt, a.M) - 1;
             const int n = last / a.span + 1;
             const size_t heads = a.K / 128, step = (size_t)a.M * heads;
-            const float2 *ml = reinterpret_cast<const float2 *>(a.ml) + blockIdx.x * heads +
+            const float2 *ml = reinterpret_cast<const float2 *>(a.ml) + row * heads +
                                col / 128;
             float m = -INFINITY, l = 0.0f;
 #pragma unroll 4
@@ -162,8 +177,10 @@ __global__ __launch_bounds__(512) void split_image_kernel(SplitArgs a) {
     auto scan = [&](int c, float4 ve, float4 vf) {
         const int o = (c >> 2) * 32 + 4 * (c & 3);
         if constexpr (SRC == SRC_PART || SRC == SRC_EMBED) {
-            *reinterpret_cast<float4 *>(a.y + base + o) = ve;
-            *reinterpret_cast<float4 *>(a.y + base + o + 16) = vf;
+            if (mine) {
+                *reinterpret_cast<float4 *>(a.y + base + o) = ve;
+                *reinterpret_cast<float4 *>(a.y + base + o + 16) = vf;
+            }
         }
         const float v[8] = {ve.x, ve.y, ve.z, ve.w, vf.x, vf.y, vf.z, vf.w};
         if constexpr (NORM) {
@@ -196,26 +213,27 @@ __global__ __launch_bounds__(512) void split_image_kernel(SplitArgs a) {
         scan(c, e, f);
     }
 #pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) {
+    for (int off = 32; off >= R; off >>= 1) {
         if constexpr (NORM) ss += __shfl_xor(ss, off);
         mx = fmaxf(mx, __shfl_xor(mx, off));
     }
-    if (lane == 0) {
-        red[0][wave] = ss;
-        red[1][wave] = mx;
+    if (lane < R) {
+        red[0][wave][ri] = ss;
+        red[1][wave][ri] = mx;
     }
     __syncthreads();
-    ss = red[0][0];
-    mx = red[1][0];
-    for (int w = 1; w < nt / 64; ++w) {
-        ss += red[0][w];
-        mx = fmaxf(mx, red[1][w]);
+    ss = red[0][0][ri];
+    mx = red[1][0][ri];
+    for (int w = 1; w < (int)blockDim.x / 64; ++w) {
+        ss += red[0][w][ri];
+        mx = fmaxf(mx, red[1][w][ri]);
     }
+    if (!mine) return;
     const float inv = NORM ? 1.0f / sqrtf(ss / (float)a.K + a.eps) : 1.0f;
     mx *= inv;
     const int e = mx > 0.0f ? max(ilogbf(mx) - 10, -126) : 0;
     const float sc = ldexpf(1.0f, -e);
-    if (tid == 0) a.rowscale[blockIdx.y * gridDim.x + blockIdx.x] = ldexpf(1.0f, e);
+    if (tid == 0) a.rowscale[blockIdx.y * a.M + row] = ldexpf(1.0f, e);
     auto emit = [&](int c, float4 ve, float4 vf) {
         const int b = c >> 2, g = c & 3;
         float v[8] = {ve.x, ve.y, ve.z, ve.w, vf.x, vf.y, vf.z, vf.w};
@@ -235,10 +253,10 @@ __global__ __launch_bounds__(512) void split_image_kernel(SplitArgs a) {
             hb[k] = __builtin_bit_cast(uint16_t, h);
             lb[k] = __builtin_bit_cast(uint16_t, (_Float16)(t - (float)h));
         }
-        uint16_t *p = a.img + (((size_t)blockIdx.x * (a.K >> 5) + b) << 6) + 8 * g;
+        uint16_t *p = a.img + (((size_t)(row >> 4) * (a.K >> 5) + b) << 10) + 128 * g + 8 * (row & 15);
         *reinterpret_cast<uint4 *>(p) = make_uint4(hb[0] | hb[2] << 16, hb[4] | hb[6] << 16,
                                                    hb[1] | hb[3] << 16, hb[5] | hb[7] << 16);
-        *reinterpret_cast<uint4 *>(p + 32) = make_uint4(lb[0] | lb[2] << 16, lb[4] | lb[6] << 16,
+        *reinterpret_cast<uint4 *>(p + 512) = make_uint4(lb[0] | lb[2] << 16, lb[4] | lb[6] << 16,
                                                         lb[1] | lb[3] << 16, lb[5] | lb[7] << 16);
     };
 #pragma unroll
@@ -309,10 +327,11 @@ struct GT {
     static constexpr int BM = 16 * RT * WM, BN = 16 * CT * WN;
     static constexpr int WAVES = WM * WN, THREADS = 64 * WAVES;
     // one stage in LDS: x [row tile][block][hi | lo][lane] x 16 B, quants
-    // [column][slot] x 16 B; beside the stages, the scales of two groups of
-    // eight blocks, [column] x 16 B each
+    // [column][slot] x 16 B; beside the stages, the scales of GROUPS groups
+    // of eight blocks, [column] x 16 B each (those of the stages in flight)
     static constexpr int OQ = BM * SB * 128, BUF = OQ + BN * SB * 16;
-    static constexpr int OD = NBUF * BUF, LDS = OD + 2 * BN * 16;
+    static constexpr int GROUPS = NBUF * SB > 12 ? 4 : 2;
+    static constexpr int OD = NBUF * BUF, LDS = OD + GROUPS * BN * 16;
     // 64-lane DMAs: of one stage by kind (a wave issues PX + PQ of them), and
     // of one group's scales (PD each by the first DW waves)
     static constexpr int NX = BM / 16 * SB * 2, NQ = BN * SB / 64, ND = BN / 64;
@@ -321,6 +340,7 @@ struct GT {
     static_assert(NX % WAVES == 0 && NQ % WAVES == 0 && ND % DW == 0 && BN % 64 == 0,
                   "every wave issues whole DMAs");
     static_assert(8 % SB == 0, "a group is whole stages");
+    static_assert(NBUF <= 3 || (NBUF - 2) * SB == 8, "one new group among the stages in flight");
     static_assert(LDS <= 160 * 1024, "LDS");
     static_assert((NBUF - 1) * PENDING + PD < 64, "wait count");
 };
@@ -445,46 +465,61 @@ void q4_gemm_kernel(cwi::GemmArgs a, int MT, int NT, int S, int per) {
     const int kb0 = min(nb, sp * per), kb1 = min(nb, kb0 + per);
     const int n_st = (kb1 - kb0 + SB - 1) / SB;
 
-    // ---- the DMAs' lane offsets (bytes) from each kind's uniform base
-    const uint32_t xo = ((uint32_t)li * nb * 8 + lg) * 16;
+    // ---- the DMAs: sources from the stage's first block, which the stage
+    // adds as one uniform offset (the address arithmetic of a stage is then a
+    // handful of scalar adds).  Rows past N re-read the last.
     const int q_row = lane / SB, q_slot = lane % SB;
     const char *const img = reinterpret_cast<const char *>(a.img) + (size_t)m0 * nb * 128;
+    uint32_t xo[G::PX], qo[G::PQ];
+    const uint8_t *qb[G::PQ];  // (SwiGLU: the matrix of each DMA)
+    const uint16_t *ds[G::PD];
+#pragma unroll
+    for (int p = 0; p < G::PX; ++p) {
+        const int u = wave + p * G::WAVES;
+        const int t = u / (2 * SB), b = u / 2 % SB, half = u & 1;
+        xo[p] = ((uint32_t)t * nb + b) * 2048 + half * 1024 + lane * 16;
+    }
+#pragma unroll
+    for (int p = 0; p < G::PQ; ++p) {
+        const int c0 = (wave + p * G::WAVES) * (64 / SB);
+        bool up;
+        const int r = min(n0 + w_row<SWI, G>(c0 + q_row, &up), a.N - 1) - n0;
+        qo[p] = ((uint32_t)r * nb + (q_slot ^ swz<SB>(c0 + q_row))) * 16;
+        if constexpr (!(SWI && CT % 2)) (void)w_row<SWI, G>(c0, &up);  // (one matrix per DMA)
+        qb[p] = (up ? a.qB : a.qA) + (size_t)n0 * nb * 16;
+    }
+#pragma unroll
+    for (int p = 0; p < G::PD; ++p) {
+        bool up;
+        const int r = min(n0 + w_row<SWI, G>((wave + p * G::DW) * 64 + lane, &up), a.N - 1);
+        ds[p] = (up ? a.sB : a.sA) + (size_t)r * ns;
+    }
     auto issue = [&](int st, unsigned char *buf) {
         const int kb = kb0 + st * SB;
-        const int lim = nb - 1 - kb;  // blocks past the row's end re-read its last
+        // blocks past the row's end (its last stage only) re-read its last
+        const int over = kb + SB - nb;
 #pragma unroll
         for (int p = 0; p < G::PX; ++p) {
-            const int u = wave + p * G::WAVES;
-            const int t = u / (2 * SB), b = u / 2 % SB, half = u & 1;
-            dma16(img + ((size_t)(16 * t) * nb + kb + min(b, lim)) * 128 + half * 64, xo,
-                  buf + u * 1024);
+            const int u = wave + p * G::WAVES, b = u / 2 % SB;
+            const uint32_t back = over > 0 ? max(b - (SB - 1 - over), 0) * 2048u : 0u;
+            dma16(img + (size_t)kb * 2048, xo[p] - back, buf + u * 1024);
         }
 #pragma unroll
         for (int p = 0; p < G::PQ; ++p) {
             const int u = wave + p * G::WAVES;
-            const int c0 = u * (64 / SB);
-            bool up;
-            // rows past N re-read the last
-            const int r = min(n0 + w_row<SWI, G>(c0 + q_row, &up), a.N - 1) - n0;
-            const int b = min(q_slot ^ swz<SB>(c0 + q_row), lim);
-            const size_t at = ((size_t)n0 * nb + kb) * 16;
-            const uint32_t off = ((uint32_t)r * nb + b) * 16;
-            if constexpr (SWI && CT % 2) {
-                dma16v((up ? a.qB : a.qA) + at + off, buf + G::OQ + u * 1024);
-            } else {
-                (void)w_row<SWI, G>(c0, &up);  // (one matrix per DMA)
-                dma16((up ? a.qB : a.qA) + at, off, buf + G::OQ + u * 1024);
+            uint32_t o = qo[p];
+            if (over > 0) {
+                const int b = q_slot ^ swz<SB>(u * (64 / SB) + q_row);
+                o -= max(b - (SB - 1 - over), 0) * 16;
             }
+            if constexpr (SWI && CT % 2) dma16v(qb[p] + (size_t)kb * 16 + o, buf + G::OQ + u * 1024);
+            else dma16(qb[p] + (size_t)kb * 16, o, buf + G::OQ + u * 1024);
         }
         if (kb % 8 == 0 && wave < G::DW) {  // the scales of a new group
 #pragma unroll
-            for (int p = 0; p < G::PD; ++p) {
-                const int u = wave + p * G::DW;
-                bool up;
-                const int r = min(n0 + w_row<SWI, G>(u * 64 + lane, &up), a.N - 1);
-                dma16v((up ? a.sB : a.sA) + (size_t)r * ns + kb,
-                       lds + G::OD + (kb / 8 & 1) * (BN * 16) + u * 1024);
-            }
+            for (int p = 0; p < G::PD; ++p)
+                dma16v(ds[p] + kb, lds + G::OD + (kb / 8 % G::GROUPS) * (BN * 16) +
+                                       (wave + p * G::DW) * 1024);
         }
     };
 
@@ -515,11 +550,19 @@ void q4_gemm_kernel(cwi::GemmArgs a, int MT, int NT, int S, int per) {
         if (s < n_st) issue(s, lds + s * G::BUF);
     int cur = 0;
     for (int st = 0; st < n_st; ++st) {
-        // stage st has landed: what may still fly is stage st + 1 (NBUF 3),
-        // with a group's scales when that begins one
-        if (G::NBUF == 2 || st + 1 >= n_st) wait_vm<0>();
-        else if ((kb0 + (st + 1) * SB) % 8 == 0 && wave < G::DW) wait_vm<G::PENDING + G::PD>();
-        else wait_vm<G::PENDING>();
+        // stage st has landed: what may still fly are the NBUF - 2 stages
+        // after it, with the scales of the groups that they begin
+        constexpr int AHEAD = G::NBUF - 2;
+        if (AHEAD == 0 || st + AHEAD >= n_st) {
+            wait_vm<0>();
+        } else if (AHEAD * SB % 8 == 0) {  // whole groups
+            if (wave < G::DW) wait_vm<AHEAD * G::PENDING + AHEAD * SB / 8 * G::PD>();
+            else wait_vm<AHEAD * G::PENDING>();
+        } else if ((kb0 + (st + 1) * SB) % 8 == 0 && wave < G::DW) {
+            wait_vm<AHEAD * G::PENDING + G::PD>();
+        } else {
+            wait_vm<AHEAD * G::PENDING>();
+        }
         lds_barrier();  // stage st published; stage st - 1's buffer is free
         if (st + G::NBUF - 1 < n_st) {
             int nx = cur + G::NBUF - 1;
@@ -534,7 +577,7 @@ void q4_gemm_kernel(cwi::GemmArgs a, int MT, int NT, int S, int per) {
 #pragma unroll
             for (int b = 0; b < SB / 2; ++b)
                 d[j][b] = *reinterpret_cast<const uint32_t *>(
-                    lds + cd[j] + (kb / 8 & 1) * (BN * 16) + (kb & 7) * 2 + b * 4);
+                    lds + cd[j] + (kb / 8 % G::GROUPS) * (BN * 16) + (kb & 7) * 2 + b * 4);
         // The stage as SB x CT steps.  A step runs the MFMAs of one column
         // tile of one block; beside them go the scale FMAs of the step before
         // and the dequantization of the step after, so the vector ALU works
@@ -633,12 +676,12 @@ void q4_gemm_kernel(cwi::GemmArgs a, int MT, int NT, int S, int per) {
 
 // ---------------------------------------------------------------------------
 // Tiles and K splits.  Every tile size has a cost in microseconds, a fit to
-// 1,300 timed launches (M 4..1024 over eight Qwen3 projection shapes; 7-9 %
+// 1,800 timed launches (M 4..2048 over eight Qwen3 projection shapes; 5-7 %
 // scatter): launch + blocks * (round * rounds + share * load) + mb * W +
 // part * partials, where a workgroup runs `blocks` K blocks, load is the
 // workgroups of the busiest CU, rounds is load over the occ workgroups that
 // a CU holds, and W and the partials are in MB.  The plan with the least cost
-// is within 2 % of the best of the timed ones on average (17 % at most).  The
+// is within 1.3 % of the best of the timed ones on average (23 % at most).  The
 // fit of a tile of less than 64 rows holds for one or two row tiles, which is
 // all it is used for: more of them read W again for too few rows (512 rows of
 // 4096 -> 6144 as 32 x 128 tiles: 83.7 us, as 64 x 128 in two splits 67.9).
@@ -653,12 +696,12 @@ typedef GT<2, 2, 1, 4, 4, 2> G32x128;
 typedef GT<4, 2, 1, 4, 2, 2> G64x128;
 typedef GT<4, 4, 1, 4, 2, 2> G64x256;
 constexpr Tile kTiles[] = {
-    {G16x64::BM, G16x64::BN, 4, 2.9f, 0.047f, 0.066f, 0.054f, 0.55f},
-    {G16x128::BM, G16x128::BN, 4, 3.3f, 0.081f, 0.074f, 0.088f, 0.41f},
-    {G32x64::BM, G32x64::BN, 3, 2.7f, 0.066f, 0.099f, 0.067f, 0.57f},
-    {G32x128::BM, G32x128::BN, 3, 3.8f, 0.083f, 0.133f, 0.047f, 0.54f},
-    {G64x128::BM, G64x128::BN, 3, 5.1f, 0.175f, 0.211f, 0.070f, 0.35f},
-    {G64x256::BM, G64x256::BN, 2, 8.0f, 0.274f, 0.307f, 0.054f, 0.36f},
+    {G16x64::BM, G16x64::BN, 4, 2.6f, 0.053f, 0.063f, 0.047f, 0.55f},
+    {G16x128::BM, G16x128::BN, 4, 3.1f, 0.088f, 0.066f, 0.084f, 0.41f},
+    {G32x64::BM, G32x64::BN, 3, 2.7f, 0.066f, 0.077f, 0.046f, 0.50f},
+    {G32x128::BM, G32x128::BN, 3, 3.8f, 0.083f, 0.124f, 0.038f, 0.46f},
+    {G64x128::BM, G64x128::BN, 3, 5.8f, 0.169f, 0.190f, 0.027f, 0.24f},
+    {G64x256::BM, G64x256::BN, 2, 8.4f, 0.210f, 0.344f, 0.029f, 0.28f},
 };
 constexpr int kTileCount = sizeof(kTiles) / sizeof(kTiles[0]);
 constexpr int kRowPad = 64;        // the x image has whole row tiles of any size
@@ -725,10 +768,24 @@ int launch_split_image(cw_ctx *ctx, const char *label, SplitArgs a, int rows, in
     // elements stay in registers between the two passes
     a.seg = seg_blocks ? seg_blocks * 4 : a.K / 8;
     const int nt = std::min(512, (a.seg + 63) / 64 * 64);
-    const dim3 grid(rows, (a.K / 8 + a.seg - 1) / a.seg);
+    const int segs = (a.K / 8 + a.seg - 1) / a.seg;
+    a.M = rows;
+    // four rows a workgroup where that still gives every CU one, for plain rows
+    // (merging the attention chunks of 512 rows so took 16 us, 8.4 by single rows)
+    if constexpr (SRC == SRC_ROWS) {
+        if (rows >= 4 * ctx->n_cu && a.seg >= 256) {
+            const dim3 grid((rows + 3) / 4, segs);
+            if (a.seg <= 512)
+                return cwi::launch(ctx, label, split_image_kernel<NORM, SRC, 2, 4>, grid,
+                                   dim3(1024), 0, a);
+            return cwi::launch(ctx, label, split_image_kernel<NORM, SRC, 6, 4>, grid, dim3(1024),
+                               0, a);
+        }
+    }
+    const dim3 grid(rows, segs);
     if (a.seg <= nt)
-        return cwi::launch(ctx, label, split_image_kernel<NORM, SRC, 1>, grid, dim3(nt), 0, a);
-    return cwi::launch(ctx, label, split_image_kernel<NORM, SRC, 3>, grid, dim3(nt), 0, a);
+        return cwi::launch(ctx, label, split_image_kernel<NORM, SRC, 1, 1>, grid, dim3(nt), 0, a);
+    return cwi::launch(ctx, label, split_image_kernel<NORM, SRC, 3, 1>, grid, dim3(nt), 0, a);
 }
 
 }  // namespace
@@ -788,7 +845,6 @@ int launch_attn_split(cw_ctx *ctx, const AttnPrefillPlan &p, const AttnPrefillAr
     a.x = t.part;
     a.MK = (size_t)t.M * K;
     a.ml = t.ml;
-    a.M = t.M;
     a.start = t.start;
     a.pt = p.pt;
     a.span = p.ct * p.kt;
