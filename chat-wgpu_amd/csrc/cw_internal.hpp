@@ -332,6 +332,8 @@ struct GemmArgs {
 // tiles: the GEMM's DMA reads them; rows past M are never stored to y, so
 // they need no values)
 size_t gemm_img_elems(int M, int K);
+// Floats of its row scales (any number of segments).
+size_t gemm_rowscale_floats(int M);
 // padded scales of N rows of K, for matrices whose scales the GEMM cannot
 // read in pairs (0: not needed)
 size_t gemm_spad_elems(int N, int K, const void *scales);

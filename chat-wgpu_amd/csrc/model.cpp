@@ -513,7 +513,7 @@ int alloc_prefill(cw_model *m, int n) {
     CW_TRY(al((size_t)n * m->q_dim * 4, (void **)&m->pf_attn));
     CW_TRY(al((size_t)n * c.hidden * 4, (void **)&m->pf_act));
     CW_TRY(al(gemm_img_elems(n, (int)wide) * 2, (void **)&m->pf_img));
-    CW_TRY(al((size_t)n * kMaxSplits * 4, (void **)&m->pf_rowscale));
+    CW_TRY(al(gemm_rowscale_floats(n) * 4, (void **)&m->pf_rowscale));
     // split-K partials of the largest plan (for n and for shorter prompts,
     // whose plans split further), and room for padded scales
     struct Shape {

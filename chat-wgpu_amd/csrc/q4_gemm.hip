@@ -548,6 +548,13 @@ void q4_gemm_kernel(cwi::GemmArgs a, int MT, int NT, int S, int per) {
 #pragma unroll
     for (int s = 0; s < G::NBUF - 1; ++s)
         if (s < n_st) issue(s, lds + s * G::BUF);
+    // this lane's row scales, asked for before the loop (at its end their
+    // latency would stand alone; rowscale is padded to whole row tiles)
+    const float *const rsp = a.rowscale + (a.seg_blocks ? (size_t)sp * a.M : 0) + m0;
+    f32x4 rs[RT];
+#pragma unroll
+    for (int i = 0; i < RT; ++i)
+        __builtin_memcpy(&rs[i], rsp + (wm * RT + i) * 16 + 4 * lg, 16);
     int cur = 0;
     for (int st = 0; st < n_st; ++st) {
         // stage st has landed: what may still fly are the NBUF - 2 stages
@@ -632,26 +639,24 @@ void q4_gemm_kernel(cwi::GemmArgs a, int MT, int NT, int S, int per) {
         for (int r = 0; r < 4; ++r)
             acc[i][CT - 1][r] = __builtin_fmaf(dp, t[1][i][r], acc[i][CT - 1][r]);
 
-    const float *const rsp = a.rowscale + (a.seg_blocks ? (size_t)sp * a.M : 0);
     constexpr int JN = SWI ? (CT + 1) / 2 : CT;
 #pragma unroll
     for (int i = 0; i < RT; ++i)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const int m = m0 + (wm * RT + i) * 16 + 4 * lg + r;
-            const float rs = rsp[min(m, a.M - 1)];
 #pragma unroll
             for (int j = 0; j < JN; ++j) {
                 int n = n0 + (wn * JN + j) * 16 + li;
                 bool mine = true;
-                const float v = acc[i][j][r] * kUnscale * rs;
+                const float v = acc[i][j][r] * kUnscale * rs[i][r];
                 float up = 0.0f;
                 if constexpr (SWI && CT % 2) {  // lanes li < 8: gate, li + 8: up
                     n = n0 + wn * 8 + (li & 7);
                     up = __shfl_xor(v, 8);
                     mine = li < 8;
                 } else if constexpr (SWI) {
-                    up = acc[i][j + CT / 2][r] * kUnscale * rs;
+                    up = acc[i][j + CT / 2][r] * kUnscale * rs[i][r];
                 }
                 if (mine && m < a.M && n < a.N) {
                     const size_t o = (size_t)m * a.N + n;
@@ -796,6 +801,8 @@ size_t gemm_img_elems(int M, int K) {
     return (size_t)((M + kRowPad - 1) / kRowPad) * kRowPad * K * 2;
 }
 
+size_t gemm_rowscale_floats(int M) { return (size_t)M * kMaxSplits + kRowPad; }
+
 size_t gemm_spad_elems(int N, int K, const void *scales) {
     return scales_in_groups(K, scales) ? 0 : (size_t)N * ((K / 32 + 7) / 8 * 8);
 }
@@ -928,7 +935,7 @@ extern "C" int cw_q4_gemm(cw_ctx *ctx, const float *x, int m, const uint16_t *sc
     // image, row scales, padded scales, partials (each 16-byte aligned)
     const size_t part = gemm_part_floats(ctx, EPI_STORE, m, out_f, in_f);
     const size_t rs_off = gemm_img_elems(m, in_f) * 2;
-    const size_t sp_off = rs_off + (((size_t)m * 4 + 15) & ~size_t(15));
+    const size_t sp_off = rs_off + ((((size_t)m + kRowPad) * 4 + 15) & ~size_t(15));
     const size_t part_off = sp_off + ((gemm_spad_elems(out_f, in_f, scales) * 2 + 15) & ~size_t(15));
     void *scratch = nullptr;
     CW_TRY(ctx_scratch(ctx, part_off + part * 4, &scratch));
