@@ -641,7 +641,19 @@ void q4_gemm_kernel(cwi::GemmArgs a, int MT, int NT, int S, int per) {
 
     constexpr int JN = SWI ? (CT + 1) / 2 : CT;
 #pragma unroll
-    for (int i = 0; i < RT; ++i)
+    for (int i = 0; i < RT; ++i) {
+        // the residuals of a row tile in flight together (past the matrix they
+        // re-read its last row or column)
+        float res[4][JN];
+        if constexpr (EPI == cwi::EPI_ADD && OUT == 0) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+#pragma unroll
+                for (int j = 0; j < JN; ++j)
+                    res[r][j] = a.resid[(size_t)min(m0 + (wm * RT + i) * 16 + 4 * lg + r, a.M - 1) *
+                                            a.N +
+                                        min(n0 + (wn * JN + j) * 16 + li, a.N - 1)];
+        }
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const int m = m0 + (wm * RT + i) * 16 + 4 * lg + r;
@@ -669,15 +681,15 @@ void q4_gemm_kernel(cwi::GemmArgs a, int MT, int NT, int S, int per) {
                     } else if constexpr (EPI == cwi::EPI_STORE) {
                         a.y[o] = v;
                     } else if constexpr (EPI == cwi::EPI_ADD) {
-                        a.y[o] = a.resid[o] + v;
+                        a.y[o] = res[r][j] + v;
                     } else {
                         a.y[o] = silu_mul(v, up);
                     }
                 }
             }
         }
+    }
 }
-
 
 // ---------------------------------------------------------------------------
 // Tiles and K splits.  Every tile size has a cost in microseconds, a fit to
