@@ -153,34 +153,6 @@ struct same_type {
     using type = T;
 };
 
-__device__ __forceinline__ float2 add(float2 a, float2 b) {
-    return make_float2(a.x + b.x, a.y + b.y);
-}
-__device__ __forceinline__ float4 add(float4 a, float4 b) {
-    return make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w);
-}
-
-// The sum in order of the S >= 1 partials at(0), at(1), ...: four requested
-// at a time, so that no load waits for another's sum.
-template <typename At>
-__device__ __forceinline__ auto sum_parts(int S, At at) {
-    auto v = at(0);
-    int s = 1;
-    for (; s + 4 <= S; s += 4) {
-        const auto a = at(s), b = at(s + 1), c = at(s + 2), d = at(s + 3);
-        v = add(add(add(add(v, a), b), c), d);
-    }
-    if (s + 3 == S) {
-        const auto a = at(s), b = at(s + 1), c = at(s + 2);
-        return add(add(add(v, a), b), c);
-    }
-    if (s + 2 == S) {
-        const auto a = at(s), b = at(s + 1);
-        return add(add(v, a), b);
-    }
-    return s < S ? add(v, at(s)) : v;
-}
-
 // Enqueue fn on ctx->stream.  While profiling, the dispatch itself stamps a
 // pair of events at the kernel's start and end (hipExtLaunchKernel), so the
 // profile holds kernel execution time, as a kernel trace does, with no
@@ -309,7 +281,7 @@ int launch_argmax(cw_ctx *ctx, const float *logits, int n, uint32_t *out_dev, vo
 
 // ---- batched prefill (M positions per launch)
 
-// y[M][N] = x[M][K] . W[N][K]^T with x given as its split image (q4_gemm.hip)
+// y[M][N] = x[M][K] . W[N][K]^T with x given as its split image (q4_gemm.hpp)
 // and W split GGUF Q4_0; EPI_SWIGLU reads a second matrix (B) and stores
 // silu(A x) * (B x).
 struct GemmArgs {

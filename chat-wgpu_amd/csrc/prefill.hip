@@ -4,22 +4,15 @@
 // (model::generate runs P forwards, src/model/mod.rs:57-125; each forward is
 // Qwen3::forward, src/model/qwen3.rs:139-191).  This file computes the same
 // forward for M positions at once, with the linear layers as Q4_0
-// dequant-GEMMs on the matrix cores (q4_gemm.hip) and causal attention as MFMA
+// dequant-GEMMs on the matrix cores (q4_gemm.hpp) and causal attention as MFMA
 // tiles.
 //
 // Attention must match the f32 per-token path, so no operand is rounded below
 // what the reference computes with (details at the kernel).
 
-#include <cmath>
-
-#include "cw_internal.hpp"
+#include "q4_gemm.hpp"
 
 namespace {
-
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-
-constexpr int kT = 256;  // threads per workgroup (4 waves)
 
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll
@@ -55,7 +48,7 @@ __global__ __launch_bounds__(kT) void qk_rope_kv_kernel(const float *__restrict_
     const float *row = (S > 0 ? part : qkv) + row_off;
     // elements p[lane] and p[lane + 64] of row (of partial 0)
     auto val = [&](const float *p) {
-        return cwi::sum_parts(max(S, 1), [&](int s2) {
+        return sum_parts(max(S, 1), [&](int s2) {
             const float *q = p + (size_t)s2 * MN + lane;
             return make_float2(q[0], q[HALF]);
         });
@@ -112,7 +105,7 @@ __global__ __launch_bounds__(kT) void qk_rope_kv_kernel(const float *__restrict_
 // Key chunks: a workgroup takes `ct` key tiles of its rows' range, so that few
 // rows against many keys, and the long rows of a causal prompt, still spread
 // over the chip.  With more than one chunk it leaves (max, sum, o) partials,
-// which the pass that reads the rows merges (q4_gemm.hip).
+// which the pass that reads the rows merges (q4_gemm.hpp).
 template <typename KVT, int QT_>
 struct AP {
     static constexpr int QT = QT_, HD = 128, ES = (int)sizeof(KVT);
@@ -126,16 +119,6 @@ struct AP {
 
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
-typedef __attribute__((address_space(3))) unsigned char lds_u8;
-
-// 64-lane global -> LDS DMA, 16 bytes per lane: lane i's land at lds_dst +
-// 16 i (wave-uniform).  asm, so that the compiler's wait counts leave it out;
-// the kernel waits for it itself.
-__device__ __forceinline__ void dma16(const void *base, uint32_t off, unsigned char *lds_dst) {
-    const uint32_t d = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lds_u8 *)lds_dst);
-    asm volatile("global_load_lds_dwordx4 %0, %1" : : "v"(off), "s"(base), "{m0}"(d) : "memory");
-}
-
 __device__ __forceinline__ f16x8 pack_f16x8(const float (&v)[8]) {
     uint32_t p[4];
 #pragma unroll

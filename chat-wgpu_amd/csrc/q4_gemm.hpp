@@ -1,6 +1,6 @@
 // Q4_0 dequant-GEMM for gfx950: y[M][N] = x[M][K] . W[N][K]^T for several
 // activation rows at once (W split GGUF Q4_0), with the passes that prepare
-// its operand and add its K splits.
+// its operand and add its K splits.  Part of prefill.hip's translation unit.
 //
 // The reference has no batched path: its prompt phase is the per-token loop
 // (src/model/mod.rs:57-125) over q4::gemv (src/kernels/q4.rs:9-30,
@@ -29,6 +29,8 @@
 // block: lane group g = l / 16 takes bytes 4 g .. 4 g + 3 of the block, whose
 // masks yield the elements in the order kept by the x image (chunk order
 // below).
+
+#pragma once
 
 #include <cmath>
 
@@ -85,8 +87,36 @@ struct SplitArgs {
     float *rowscale;
 };
 
+__device__ __forceinline__ float2 add(float2 a, float2 b) {
+    return make_float2(a.x + b.x, a.y + b.y);
+}
+__device__ __forceinline__ float4 add(float4 a, float4 b) {
+    return make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w);
+}
+
+// The sum in order of the S >= 1 partials at(0), at(1), ...: four requested
+// at a time, so that no load waits for another's sum.
+template <typename At>
+__device__ __forceinline__ auto sum_parts(int S, At at) {
+    auto v = at(0);
+    int s = 1;
+    for (; s + 4 <= S; s += 4) {
+        const auto a = at(s), b = at(s + 1), c = at(s + 2), d = at(s + 3);
+        v = add(add(add(add(v, a), b), c), d);
+    }
+    if (s + 3 == S) {
+        const auto a = at(s), b = at(s + 1), c = at(s + 2);
+        return add(add(add(v, a), b), c);
+    }
+    if (s + 2 == S) {
+        const auto a = at(s), b = at(s + 1);
+        return add(add(v, a), b);
+    }
+    return s < S ? add(v, at(s)) : v;
+}
+
 __device__ __forceinline__ float4 sum4(const float *p, int S, size_t stride) {
-    return cwi::sum_parts(S, [&](int s) {
+    return sum_parts(S, [&](int s) {
         return *reinterpret_cast<const float4 *>(p + (size_t)s * stride);
     });
 }
