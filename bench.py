@@ -172,8 +172,8 @@ def gemv_profile(prof, n_steps):
 
 
 def bench_06b(ctx, warm=True):
-    """Qwen3-0.6B-shape token loop (32 prompt + 128 greedy, f32 KV, graph
-    replay), and the same model's Q4 GEMV launches of one decode token timed
+    """Qwen3-0.6B-shape token loop (32 prompt tokens batched, then 128 greedy,
+    f32 KV, graph replay), and the same model's Q4 GEMV launches of one decode token timed
     by kernel timestamps over 8 eager steps (the GEMVs of one 0.6B step)."""
     P, N = 32, 128
     cfg = cw.make_config(28, 1024, 16, 8, 128, 3072, 151936, P + N, cw.CW_F32, 1e-6, 1e6)
@@ -514,8 +514,8 @@ def main():
         tps06, el06, gb06, gms06, gl06 = bench_06b(ctx)
         ex = result["extras"]
         ex["qwen3_0.6b_token_loop_tok_s"] = round(tps06, 1)
-        ex["qwen3_0.6b_token_loop"] = ("32 prompt + 128 greedy, f32 KV, 159 forwards incl. "
-                                       "prompt, HIP graph")
+        ex["qwen3_0.6b_token_loop"] = ("32 prompt + 128 greedy, f32 KV, 159 forwards: the "
+                                       "prompt batched, then HIP graph replays")
         ex["qwen3_0.6b_step_gemvs"] = {
             "workload": "one Qwen3-0.6B-shape decode step's Q4_0 GEMVs (28 layers x "
                         "QKV, O, gate/up, down + LM head 1024->151936), kernel timestamps "

@@ -106,6 +106,13 @@ __global__ __launch_bounds__(kT) void qk_rope_kv_kernel(const float *__restrict_
 // rows against many keys, and the long rows of a causal prompt, still spread
 // over the chip.  With more than one chunk it leaves (max, sum, o) partials,
 // which the pass that reads the rows merges (q4_gemm.hpp).
+//
+// Bound by the softmax's vector work and waits beside short MFMA runs (512
+// positions: matrix cores busy 7 %, waves waiting 39 % of their time), so the
+// layout aims at fewer K / V reads and LDS trips.  One head per workgroup with P
+// through LDS took, per layer of 32 heads over 8: 24 positions behind 700
+// 29.2 us, 512 from 0 23.5, 3000 from 0 401; this form 10, 20 and 171, and the
+// merge 4.6, 8.7 and 28.
 template <typename KVT, int QT_>
 struct AP {
     static constexpr int QT = QT_, HD = 128, ES = (int)sizeof(KVT);

@@ -477,6 +477,16 @@ __device__ __forceinline__ int w_row(int c, bool *up) {
 // OUT: 0 = the epilogue EPI into y, 1 = f32 partials of split sp into part.
 // SwiGLU: a wave holds matching columns of both matrices, so silu(g) u is
 // formed in registers.
+//
+// Bound, at 512 rows, by the chain of dequantization, MFMAs and scale FMAs,
+// which the operands' DMAs overlap only in part (matrix cores busy 30-44 %; 4096
+// -> 6144 with row-major x: 73.7 us, 53 without DMA, 90 with DMA alone); at few
+// rows by the launch, the first loads and W at about 2.3 TB/s.  Four waves side
+// by side along N dequantize every weight once; tiles of 16 and 32 rows keep
+// few rows from paying for padding.  128 x 128 tiles with row-major x took, with the passes around them,
+// 43.2 us for 16 rows of 4096 -> 12288 (here 17.1, this kernel 40.3 -> 12.2),
+// 52.3 for 100 of 12288 -> 4096 (here 42.5), 86.5 for 512 of 4096 -> 6144 (here
+// 69.5).
 template <int EPI, int OUT, class G, int OCC>
 __global__ __launch_bounds__(G::THREADS) __attribute__((amdgpu_waves_per_eu(OCC, OCC)))
 void q4_gemm_kernel(cwi::GemmArgs a, int MT, int NT, int S, int per) {

@@ -266,6 +266,8 @@ int cw_model_tap(cw_model *m, const char *name, int layer, float *host_out, int 
 /* model::generate (src/model/mod.rs:57-125): greedy loop over the prompt then
  * max_new produced tokens (P+N-1 forwards), the whole step device-resident
  * (position and token live on the device), executed as `mode` (CW_STEP_*).
+ * In CW_STEP_GRAPH mode with head_dim 128 a prompt of two or more tokens runs
+ * as one batch (as in cw_model_prefill) and the replayed steps follow.
  * The first prompt token is fed at start_pos (0 = empty cache).  Writes
  * max_new ids to out_tokens.  CW_STEP_FUSED returns CW_ERR_ARG for shapes it
  * does not cover and CW_ERR_HIP if a grid barrier timed out. */
