@@ -312,9 +312,10 @@ size_t gemm_spad_elems(int N, int K, const void *scales);
 // floats of split-K partials the GEMM's plan takes for this shape (0: none);
 // with less room it takes the best plan that fits
 size_t gemm_part_floats(const cw_ctx *ctx, Epi epi, int M, int N, int K);
-// The split image of rows of x, RMS-normalised with norm_w when set.
+// The split image of rows of x, RMS-normalised with norm_w when set; without,
+// a row scale per seg_blocks blocks (0: per row).
 int launch_split_rows(cw_ctx *ctx, const float *x, const float *norm_w, float eps, int rows, int K,
-                      uint16_t *img, float *rowscale);
+                      uint16_t *img, float *rowscale, int seg_blocks);
 // The embedding rows of `rows` tokens (ids on the device, validated < vocab by
 // the caller) into y, and their RMS-normalised split image.
 int launch_embed_split(cw_ctx *ctx, const float *table, const uint32_t *tok_dev,

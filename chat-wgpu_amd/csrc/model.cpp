@@ -635,17 +635,15 @@ int enqueue_prefill(cw_model *m, int tok, int n, int start) {
         at.kc = kc;
         at.vc = vc;
         CW_TRY(launch_attn_prefill(ctx, plan, at, c.kv_dtype));
-        const int seg_a = plan.chunks > 1 ? seg_o : 0;
-        CW_TRY(launch_attn_split(ctx, plan, at, seg_a, m->pf_img, m->pf_rowscale));
+        CW_TRY(launch_attn_split(ctx, plan, at, seg_o, m->pf_img, m->pf_rowscale));
         CW_TRY(pf_gemm(m, n, m->q_dim, EPI_ADD, L.wo, nullptr, m->pf_hidden, m->pf_hidden, &g,
-                       &splits, seg_a));
+                       &splits, seg_o));
         CW_TRY(to_image(EPI_ADD, g, splits, L.ffn_norm, 0));
         CW_TRY(tap_row(m, m->tap_post + (size_t)i * c.dim, m->pf_hidden, n - 1, c.dim));
         CW_TRY(pf_gemm(m, n, c.dim, EPI_SWIGLU, L.gate, &L.up, nullptr, m->pf_act, &g, &splits));
-        const int seg_h = splits ? seg_d : 0;
-        CW_TRY(to_image(EPI_SWIGLU, g, splits, nullptr, seg_h));
+        CW_TRY(to_image(EPI_SWIGLU, g, splits, nullptr, seg_d));
         CW_TRY(pf_gemm(m, n, c.hidden, EPI_ADD, L.down, nullptr, m->pf_hidden, m->pf_hidden, &g,
-                       &splits, seg_h));
+                       &splits, seg_d));
         if (i + 1 < c.n_layers)
             CW_TRY(to_image(EPI_ADD, g, splits, m->layers[i + 1].attn_norm, 0));
         else if (splits)

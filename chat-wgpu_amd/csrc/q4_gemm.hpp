@@ -59,7 +59,7 @@ constexpr float kUnscale = 0.0625f;  // the products' factor 16
 // One workgroup per row, or per (row, segment of the columns) with a row scale
 // for each: where the consumer splits K by the same segments, few long rows
 // still give every CU a workgroup (the SwiGLU pass of 24 rows of 12288: 15.6
-// us as 24 workgroups).  RMSNorm needs whole rows.  A thread takes whole
+// us as 24 workgroups, 5.0 so).  RMSNorm needs whole rows.  A thread takes whole
 // chunks (8 elements), CH of them in registers.  Sources of a row: SRC_ROWS, x itself; SRC_PART, the sum in
 // order of S split-K partials (+ resid), also written to y; SRC_SWIGLU,
 // silu(g) u of the summed partials of the gate and the up product; SRC_EMBED,
@@ -484,9 +484,9 @@ __device__ __forceinline__ int w_row(int c, bool *up) {
 // rows by the launch, the first loads and W at about 2.3 TB/s.  Four waves side
 // by side along N dequantize every weight once; tiles of 16 and 32 rows keep
 // few rows from paying for padding.  128 x 128 tiles with row-major x took, with the passes around them,
-// 43.2 us for 16 rows of 4096 -> 12288 (here 17.1, this kernel 40.3 -> 12.2),
-// 52.3 for 100 of 12288 -> 4096 (here 42.5), 86.5 for 512 of 4096 -> 6144 (here
-// 69.5).
+// 43.1 us for 16 rows of 4096 -> 12288 (here 16.5, this kernel 40.3 -> 11.5),
+// 52.2 for 100 of 12288 -> 4096 (here 41.5), 86.5 for 512 of 4096 -> 6144 (here
+// 69.6).
 template <int EPI, int OUT, class G, int OCC>
 __global__ __launch_bounds__(G::THREADS) __attribute__((amdgpu_waves_per_eu(OCC, OCC)))
 void q4_gemm_kernel(cwi::GemmArgs a, int MT, int NT, int S, int per) {
@@ -827,10 +827,13 @@ int launch_split_image(cw_ctx *ctx, const char *label, SplitArgs a, int rows, in
     const int nt = std::min(512, (a.seg + 63) / 64 * 64);
     const int segs = (a.K / 8 + a.seg - 1) / a.seg;
     a.M = rows;
-    // four rows a workgroup where that still gives every CU one, for plain rows
+    // four rows a workgroup where that still gives every CU one, for plain rows;
+    // counted with a row's segments only above 256 chunks each (512 rows of 12288
+    // in four: 9.9 us, 13.4 by single rows; of 4096 in two: 7.1 against 6.1)
     // (merging the attention chunks of 512 rows so took 16 us, 8.4 by single rows)
     if constexpr (SRC == SRC_ROWS) {
-        if (rows >= 4 * ctx->n_cu && a.seg >= 256) {
+        if ((rows >= 4 * ctx->n_cu && a.seg >= 256) ||
+            (rows * segs >= 4 * ctx->n_cu && a.seg > 256)) {
             const dim3 grid((rows + 3) / 4, segs);
             if (a.seg <= 512)
                 return cwi::launch(ctx, label, split_image_kernel<NORM, SRC, 2, 4>, grid,
@@ -869,7 +872,7 @@ int gemm_seg_blocks(const cw_ctx *ctx, Epi epi, int M, int N, int K, size_t part
 }
 
 int launch_split_rows(cw_ctx *ctx, const float *x, const float *norm_w, float eps, int rows, int K,
-                      uint16_t *img, float *rowscale) {
+                      uint16_t *img, float *rowscale, int seg_blocks) {
     SplitArgs a{};
     a.x = x;
     a.norm_w = norm_w;
@@ -878,7 +881,7 @@ int launch_split_rows(cw_ctx *ctx, const float *x, const float *norm_w, float ep
     a.img = img;
     a.rowscale = rowscale;
     return norm_w ? launch_split_image<true, SRC_ROWS>(ctx, "prefill_split_rmsnorm", a, rows)
-                  : launch_split_image<false, SRC_ROWS>(ctx, "prefill_split", a, rows);
+                  : launch_split_image<false, SRC_ROWS>(ctx, "prefill_split", a, rows, seg_blocks);
 }
 
 int launch_embed_split(cw_ctx *ctx, const float *table, const uint32_t *tok_dev,
@@ -899,7 +902,8 @@ int launch_embed_split(cw_ctx *ctx, const float *table, const uint32_t *tok_dev,
 int launch_attn_split(cw_ctx *ctx, const AttnPrefillPlan &p, const AttnPrefillArgs &t,
                       int seg_blocks, uint16_t *img, float *rowscale) {
     const int K = t.n_heads * 128;
-    if (p.chunks == 1) return launch_split_rows(ctx, t.out, nullptr, 0.0f, t.M, K, img, rowscale);
+    if (p.chunks == 1)
+        return launch_split_rows(ctx, t.out, nullptr, 0.0f, t.M, K, img, rowscale, seg_blocks);
     SplitArgs a{};
     a.x = t.part;
     a.MK = (size_t)t.M * K;
@@ -963,7 +967,8 @@ int launch_reduce_split(cw_ctx *ctx, Epi epi, const GemmArgs &g, int splits, con
     a.K = g.N;
     a.img = img;
     a.rowscale = rowscale;
-    if (!splits) return launch_split_rows(ctx, g.y, norm_w, eps, g.M, g.N, img, rowscale);
+    if (!splits)
+        return launch_split_rows(ctx, g.y, norm_w, eps, g.M, g.N, img, rowscale, seg_blocks);
     if (epi == EPI_SWIGLU)
         return launch_split_image<false, SRC_SWIGLU>(ctx, "q4_gemm_reduce_swiglu", a, g.M,
                                                      seg_blocks);
@@ -987,7 +992,7 @@ extern "C" int cw_q4_gemm(cw_ctx *ctx, const float *x, int m, const uint16_t *sc
     // image, row scales, padded scales, partials (each 16-byte aligned)
     const size_t part = gemm_part_floats(ctx, EPI_STORE, m, out_f, in_f);
     const size_t rs_off = gemm_img_elems(m, in_f) * 2;
-    const size_t sp_off = rs_off + ((((size_t)m + kRowPad) * 4 + 15) & ~size_t(15));
+    const size_t sp_off = rs_off + ((gemm_rowscale_floats(m) * 4 + 15) & ~size_t(15));
     const size_t part_off = sp_off + ((gemm_spad_elems(out_f, in_f, scales) * 2 + 15) & ~size_t(15));
     void *scratch = nullptr;
     CW_TRY(ctx_scratch(ctx, part_off + part * 4, &scratch));
@@ -995,7 +1000,8 @@ extern "C" int cw_q4_gemm(cw_ctx *ctx, const float *x, int m, const uint16_t *sc
     GemmArgs a{};
     uint16_t *img = reinterpret_cast<uint16_t *>(base);
     float *rs = reinterpret_cast<float *>(base + rs_off);
-    CW_TRY(launch_split_rows(ctx, x, nullptr, 0.0f, m, in_f, img, rs));
+    a.seg_blocks = part ? gemm_seg_blocks(ctx, EPI_STORE, m, out_f, in_f, part) : 0;
+    CW_TRY(launch_split_rows(ctx, x, nullptr, 0.0f, m, in_f, img, rs, a.seg_blocks));
     a.img = img;
     a.rowscale = rs;
     a.sA = scales;

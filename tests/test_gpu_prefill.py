@@ -51,7 +51,8 @@ def test_q4_gemm_vs_oracle(ctx, m, in_f, out_f):
 # its scale groups (8 blocks) and K splits, one row and one column included
 GEMM_EDGES = [(m, k, n) for m in (1, 15, 17, 33, 63, 65, 129)
               for k, n in ((32, 1), (288, 63), (2048, 129))] + \
-             [(2, 12288, 65), (16, 40960, 64), (31, 4128, 257), (260, 1024, 300)]
+             [(2, 12288, 65), (16, 40960, 64), (31, 4128, 257), (260, 1024, 300),
+              (513, 12288, 4096)]
 
 
 @pytest.mark.parametrize("m,in_f,out_f", GEMM_EDGES)
