@@ -18,10 +18,11 @@
 //    times their x (below 2^15), so every product has the factor 16.  (The
 //    masked nibble alone is q as an f16 subnormal, with no or and no
 //    subtraction, but the matrix cores align products by their nominal
-//    exponents: 1.6e-5 relative error in y where this form has 1.5e-7.)
+//    exponents: 1.6e-5 relative error in y where this form has 1.0-1.4e-7.)
 // Per block b: t = sum over its 32 k of (x_hi + x_lo) (q - 8), two MFMAs into
 // a fresh f32 accumulator, then acc += d_b t, one f32 FMA per output element
-// and block; y = 2^(e - 4) acc.
+// and block; every kChain blocks acc is added to a second sum and starts again
+// (the kernel's comment); y = 2^(e - 4) of that sum.
 //
 // MFMA v_mfma_f32_16x16x32_f16: lane l holds A[l % 16][8 (l / 16) + j] and
 // B[8 (l / 16) + j][l % 16] (j = 0..7) and receives D[4 (l / 16) + r][l % 16]
@@ -45,6 +46,7 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kT = 256;
 constexpr float kUnscale = 0.0625f;  // the products' factor 16
+constexpr int kChain = 16;           // blocks per chain of f32 sums (a multiple of every stage)
 
 // ---------------------------------------------------------------------------
 // The x image: per 16 rows and block 1 KB of x_hi, then 1 KB of x_lo, each as
@@ -369,7 +371,8 @@ struct GT {
     static constexpr int DW = ND < WAVES ? ND : WAVES, PD = ND / DW;
     static_assert(NX % WAVES == 0 && NQ % WAVES == 0 && ND % DW == 0 && BN % 64 == 0,
                   "every wave issues whole DMAs");
-    static_assert(8 % SB == 0, "a group is whole stages");
+    static_assert(8 % SB == 0 && kChain % 8 == 0, "groups and chains are whole stages");
+    static_assert(BM <= 64 && WM == 1, "a lane holds a row's scale");
     static_assert(NBUF <= 3 || (NBUF - 2) * SB == 8, "one new group among the stages in flight");
     static_assert(LDS <= 160 * 1024, "LDS");
     static_assert((NBUF - 1) * PENDING + PD < 64, "wait count");
@@ -478,6 +481,15 @@ __device__ __forceinline__ int w_row(int c, bool *up) {
 // SwiGLU: a wave holds matching columns of both matrices, so silu(g) u is
 // formed in registers.
 //
+// Sums: a chain of n additions has an error of about sqrt(n) roundings, so
+// chains end after kChain blocks, whatever the plan's K splits.  Error against
+// 64 bits (2-norm) with 2 to 3000 rows: 4096 -> 6144 1.1-1.2e-7 (one chain of
+// 128 blocks 2.1e-7, four of 32 1.3e-7), 12288 -> 4096 1.2-1.4e-7 (one of 384
+// 3.6e-7), 1024 -> 3072 0.9-1.0e-7; q4_gemv.hip's f32 products have 1.7-2.2e-7.
+// (x_lo's MFMA before x_hi's: 1.5e-7 for 12288.)  The second sums and the
+// additions cost 64-row tiles 0-1 % (512 rows of 4096 -> 6144 70.4 -> 70.6 us;
+// 3000-token prompts 1-2 %).
+//
 // Bound, at 512 rows, by the chain of dequantization, MFMAs and scale FMAs,
 // which the operands' DMAs overlap only in part (matrix cores busy 30-44 %; 4096
 // -> 6144 with row-major x: 73.7 us, 53 without DMA, 90 with DMA alone); at few
@@ -507,7 +519,8 @@ void q4_gemm_kernel(cwi::GemmArgs a, int MT, int NT, int S, int per) {
 
     // ---- the DMAs: sources from the stage's first block, which the stage
     // adds as one uniform offset (the address arithmetic of a stage is then a
-    // handful of scalar adds).  Rows past N re-read the last.
+    // handful of scalar adds; xo is uniform, a lane adds only its 16 bytes).
+    // Rows past N re-read the last.
     const int q_row = lane / SB, q_slot = lane % SB;
     const char *const img = reinterpret_cast<const char *>(a.img) + (size_t)m0 * nb * 128;
     uint32_t xo[G::PX], qo[G::PQ];
@@ -517,7 +530,7 @@ void q4_gemm_kernel(cwi::GemmArgs a, int MT, int NT, int S, int per) {
     for (int p = 0; p < G::PX; ++p) {
         const int u = wave + p * G::WAVES;
         const int t = u / (2 * SB), b = u / 2 % SB, half = u & 1;
-        xo[p] = ((uint32_t)t * nb + b) * 2048 + half * 1024 + lane * 16;
+        xo[p] = ((uint32_t)t * nb + b) * 2048 + half * 1024;
     }
 #pragma unroll
     for (int p = 0; p < G::PQ; ++p) {
@@ -542,7 +555,7 @@ void q4_gemm_kernel(cwi::GemmArgs a, int MT, int NT, int S, int per) {
         for (int p = 0; p < G::PX; ++p) {
             const int u = wave + p * G::WAVES, b = u / 2 % SB;
             const uint32_t back = over > 0 ? max(b - (SB - 1 - over), 0) * 2048u : 0u;
-            dma16(img + (size_t)kb * 2048, xo[p] - back, buf + u * 1024);
+            dma16(img + (size_t)kb * 2048 + (xo[p] - back), lane * 16, buf + u * 1024);
         }
 #pragma unroll
         for (int p = 0; p < G::PQ; ++p) {
@@ -575,28 +588,38 @@ void q4_gemm_kernel(cwi::GemmArgs a, int MT, int NT, int S, int per) {
     }
     const int xr = wm * RT * SB * 2048 + lane * 16;
 
-    f32x4 acc[RT][CT], t[2][RT];
+    f32x4 acc[RT][CT], sum[RT][CT], t[2][RT];
     float dp = 0.0f;
 #pragma unroll
     for (int i = 0; i < RT; ++i) {
         t[0][i] = t[1][i] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int j = 0; j < CT; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int j = 0; j < CT; ++j) acc[i][j] = sum[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
     static_assert(SB * CT % 2 == 0, "steps alternate between two sets of sums, tile CT - 1 last in the second");
 
 #pragma unroll
     for (int s = 0; s < G::NBUF - 1; ++s)
         if (s < n_st) issue(s, lds + s * G::BUF);
-    // this lane's row scales, asked for before the loop (at its end their
-    // latency would stand alone; rowscale is padded to whole row tiles)
-    const float *const rsp = a.rowscale + (a.seg_blocks ? (size_t)sp * a.M : 0) + m0;
-    f32x4 rs[RT];
+    // the tile's row scales, one row per lane, asked for before the loop (at
+    // its end their latency would stand alone; rowscale is padded to whole row
+    // tiles); the epilogue fetches those of its rows from the other lanes
+    const float rs = a.rowscale[(a.seg_blocks ? (size_t)sp * a.M : 0) + m0 + lane % BM];
+    // the chain of the last kChain blocks ends; a 64-row tile folds ahead of
+    // a stage, where its registers suffice without a spill, a smaller one
+    // after it (16 rows of 4096 -> 12288 16.5 us, 16.9 folding ahead)
+    auto fold = [&] {
 #pragma unroll
-    for (int i = 0; i < RT; ++i)
-        __builtin_memcpy(&rs[i], rsp + (wm * RT + i) * 16 + 4 * lg, 16);
+        for (int i = 0; i < RT; ++i)
+#pragma unroll
+            for (int j = 0; j < CT; ++j) {
+                sum[i][j] += acc[i][j];
+                acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+            }
+    };
     int cur = 0;
     for (int st = 0; st < n_st; ++st) {
+        if (RT >= 4 && st != 0 && st % (kChain / SB) == 0) fold();
         // stage st has landed: what may still fly are the NBUF - 2 stages
         // after it, with the scales of the groups that they begin
         constexpr int AHEAD = G::NBUF - 2;
@@ -672,12 +695,14 @@ void q4_gemm_kernel(cwi::GemmArgs a, int MT, int NT, int S, int per) {
             }
         }
         cur = cur + 1 == G::NBUF ? 0 : cur + 1;
+        if (RT < 4 && (st + 1) % (kChain / SB) == 0) fold();
     }
 #pragma unroll
     for (int i = 0; i < RT; ++i)
 #pragma unroll
         for (int r = 0; r < 4; ++r)
             acc[i][CT - 1][r] = __builtin_fmaf(dp, t[1][i][r], acc[i][CT - 1][r]);
+    fold();
 
     constexpr int JN = SWI ? (CT + 1) / 2 : CT;
 #pragma unroll
@@ -696,19 +721,20 @@ void q4_gemm_kernel(cwi::GemmArgs a, int MT, int NT, int S, int per) {
         }
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            const int m = m0 + (wm * RT + i) * 16 + 4 * lg + r;
+            const int mi = (wm * RT + i) * 16 + 4 * lg + r, m = m0 + mi;
+            const float sc = kUnscale * __shfl(rs, mi);
 #pragma unroll
             for (int j = 0; j < JN; ++j) {
                 int n = n0 + (wn * JN + j) * 16 + li;
                 bool mine = true;
-                const float v = acc[i][j][r] * kUnscale * rs[i][r];
+                const float v = sum[i][j][r] * sc;
                 float up = 0.0f;
                 if constexpr (SWI && CT % 2) {  // lanes li < 8: gate, li + 8: up
                     n = n0 + wn * 8 + (li & 7);
                     up = __shfl_xor(v, 8);
                     mine = li < 8;
                 } else if constexpr (SWI) {
-                    up = acc[i][j + CT / 2][r] * kUnscale * rs[i][r];
+                    up = sum[i][j + CT / 2][r] * sc;
                 }
                 if (mine && m < a.M && n < a.N) {
                     const size_t o = (size_t)m * a.N + n;

@@ -83,6 +83,28 @@ def test_q4_gemm_scales_at_odd_addresses(ctx):
     assert np.array_equal(ref, ctx.q4_gemm(x, m, at2, qd, in_f, out_f).download())
 
 
+@pytest.mark.parametrize("m,in_f,out_f", [(2, 4096, 4096), (60, 4096, 4096), (384, 4096, 12288),
+                                          (1000, 4096, 6144), (700, 12288, 4096),
+                                          (1500, 12288, 4096)])
+def test_q4_gemm_error_whatever_the_k_splits(ctx, m, in_f, out_f):
+    """The 2-norm error of sampled rows against 64 bits, for plans that split K
+    much (few rows) and not at all (many).  With one rounding of 2^-24 at most
+    per f32 sum, uniform in size (variance 2^-48 / 3, half of it over a binade)
+    and relative to a random walk's partial sum, chains of 16 blocks and the
+    sum of the chains have the variance 2^-48 / 6 (16 + blocks / 16) / 2; the
+    operands and block sums add (0.8e-7)^2 (measured at one block).  The bound
+    is 1.25 times that; one chain over all of K had 1.8 to 2.6 times."""
+    s, q = cw.synth_q4(cw.synth_key(27, f"c{out_f}x{in_f}"), out_f, in_f, 0.02)
+    x = cw.synth_normal_f32(cw.synth_key(27, f"cx{m}x{in_f}"), m * in_f).reshape(m, in_f)
+    y = ctx.q4_gemm(ctx.storage(x), m, ctx.storage(s), ctx.storage(q), in_f, out_f).download()
+    rows = np.unique(np.linspace(0, m - 1, 24).astype(int))
+    w = orc.dequant_q4_0_soa(s, q).reshape(out_f, in_f).astype(np.float64)
+    ref = x[rows].astype(np.float64) @ w.T
+    err = np.linalg.norm(y.reshape(m, out_f)[rows] - ref) / np.linalg.norm(ref)
+    var = 2.0 ** -48 / 6 * (16 + in_f / 512) / 2 + 0.8e-7 ** 2
+    assert err <= 1.25 * var ** 0.5, (err, var ** 0.5)
+
+
 # the four projection shapes of one 8B layer at the 512-token workload:
 # QKV (4096 -> 6144), O (4096 -> 4096), gate/up (4096 -> 12288, each) and
 # down (12288 -> 4096); (m, in_f, out_f).  These run the split-K and tile
