@@ -7,8 +7,8 @@
 // dequant-GEMMs on the matrix cores (q4_gemm.hpp) and causal attention as MFMA
 // tiles.
 //
-// Attention must match the f32 per-token path, so no operand is rounded below
-// what the reference computes with (details at the kernel).
+// Attention must match the f32 per-token path, so q and the softmax weights go
+// through the matrix cores as two f16 or as f32 (details at the kernel).
 
 #include "q4_gemm.hpp"
 
@@ -98,7 +98,12 @@ __global__ __launch_bounds__(kT) void qk_rope_kv_kernel(const float *__restrict_
 // shared by A and B is valid).  So P never goes through LDS, and a row's
 // scale is one value per lane.
 //  * f16 cache: v_mfma_f32_16x16x32_f16, K and V as stored, q and P split into
-//    f16 hi + lo (22 significant bits); V^T by LDS transpose loads.
+//    f16 hi + lo: 22 significant bits of what is at least 2^-3 (hi is 2^-3 or
+//    more, lo's last place is 2^-24), steps of 2^-24 below.  P is scaled by
+//    2^15, so weights down to 2^-18 of the largest keep 22 bits (unscaled, one
+//    12 nats below it kept seven: logits 2-4e-3 off behind such a key); q is
+//    RMS-normalised times a gain, as the decode kernel splits it.  V^T by LDS
+//    transpose loads.
 //  * f32 cache: v_mfma_f32_16x16x4_f32 (lane l: A[l % 16][l / 16],
 //    B[l / 16][l % 16]), every operand f32.
 //
@@ -122,6 +127,9 @@ struct AP {
     static constexpr int TILE = KT * ROWB;     // bytes of one K (or V) tile
     static constexpr int UNITS = TILE / 1024;  // 64-lane DMAs of one tile
     static constexpr int ST = KT / 16;         // score tiles of 16 keys
+    // weights carry 2^UP (which cancels in o / sum), so that small ones keep
+    // their bits as f16: the largest is 2^15, and f16 ends at 2^16 and 2^-24
+    static constexpr float UP = ES == 2 ? 15.0f : 0.0f;
 };
 
 typedef short s16x4 __attribute__((ext_vector_type(4)));
@@ -185,7 +193,7 @@ __global__ __launch_bounds__(kT, 2) void attn_prefill_kernel(cwi::AttnPrefillArg
     load_tile(t0, lds[0]);
 
     // q operands of this lane's queries (B: query li, dims in the k order of
-    // the K fragments), times scale log2(e): p = 2^(s - max)
+    // the K fragments)
     f16x8 qh[F16 ? QT : 1][4], ql[F16 ? QT : 1][4];
     f32x4 qf[F16 ? 1 : QT][8];
 #pragma unroll
@@ -291,7 +299,8 @@ __global__ __launch_bounds__(kT, 2) void attn_prefill_kernel(cwi::AttnPrefillArg
             mx = fmaxf(mx, __shfl_xor(mx, 16));
             mx = fmaxf(mx, __shfl_xor(mx, 32));
             const float mnew = fmaxf(mrow[i], mx * a.scale);
-            // a query with no key yet keeps max -inf: its terms are 2^-inf = 0
+            // p = 2^(s scale log2(e) - max + UP); a query with no key yet keeps
+            // max -inf: its terms are 2^-inf = 0
             const float ref = mnew == -INFINITY ? 0.0f : mnew;
             alpha[i] = __builtin_amdgcn_exp2f(mrow[i] - ref);
             grew |= mnew > mrow[i];
@@ -302,7 +311,7 @@ __global__ __launch_bounds__(kT, 2) void attn_prefill_kernel(cwi::AttnPrefillArg
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
                     const float p =
-                        __builtin_amdgcn_exp2f(__builtin_fmaf(s[i][kt][r], a.scale, -ref));
+                        __builtin_amdgcn_exp2f(__builtin_fmaf(s[i][kt][r], a.scale, C::UP - ref));
                     s[i][kt][r] = p;
                     ls += p;
                 }

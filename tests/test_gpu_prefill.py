@@ -424,6 +424,44 @@ def test_prefill_attention_chunks(ctx, kv, n_heads, n_kv):
     m.close()
 
 
+@pytest.mark.parametrize("n_heads,n_kv", [(4, 2), (4, 1)])
+@pytest.mark.parametrize("start,P", [(60, 3), (60, 40), (400, 3), (400, 40)])
+def test_prefill_attention_behind_a_sink(ctx, n_heads, n_kv, start, P):
+    """One key 12 to 16 nats above all others whose V row is zero, the other
+    rows of its key tile large: the output is the sum of the small softmax
+    weights, which must keep their bits, for one and two query tiles a wave and
+    with the keys in one chunk and in many.  Logits within 2e-5 of their size
+    of the oracle's f32 attention (f32 sums over some hundred keys have about
+    1e-6; f16 weights without a factor had 2e-3 to 4e-3 at 12 nats)."""
+    cfg = cw.make_config(1, 256, n_heads, n_kv, 128, 512, 500, 460, cw.CW_F16, 1e-6, 1e6)
+    weights = cw.synthetic_weights(cfg, 87)
+    prompt = cw.synth_tokens(cw.synth_key(87, f"s{start}x{P}"), P, cfg.vocab)
+    m = cw.Model(ctx, cfg)
+    m.set_weights(weights)
+    m.finalize()
+    m.set_taps(True)
+    m.prefill(prompt, start_pos=start)
+    q = m.tap("q", 0).reshape(n_kv, n_heads // n_kv, 128).astype(np.float64)
+    rng = np.random.default_rng(87)
+    for nats in (12.0, 14.0, 16.0):
+        k = (0.1 * rng.standard_normal((1, start, n_kv, 128))).astype(np.float16)
+        v = np.zeros((1, start, n_kv, 128), np.float16)
+        v[0, 1:60] = rng.uniform(-6e4, 6e4, (59, n_kv, 128))
+        for g in range(n_kv):  # the shortest key that gives all of its heads the score
+            k[0, 0, g] = np.linalg.lstsq(q[g], np.full(n_heads // n_kv, nats * 128 ** 0.5),
+                                         rcond=None)[0]
+        bits = [x.reshape(1, start, -1).view(np.uint16) for x in (k, v)]
+        m.prefill_kv(*bits, start)
+        m.prefill(prompt, start_pos=start)
+        o = orc.OracleModel(cfg, weights)
+        o.prefill_kv(*bits, start)
+        ref = oracle_prompt_logits(o, prompt, start)
+        o.close()
+        err = float(np.max(np.abs(m.logits() - ref)) / np.max(np.abs(ref)))
+        assert err <= 2e-5, (nats, err)
+    m.close()
+
+
 @pytest.mark.parametrize("kv", [cw.CW_F16, cw.CW_F32])
 @pytest.mark.parametrize("P,start", [(1, 0), (3, 0), (4, 0), (37, 0), (5, 20)])
 def test_generate_batches_its_prompt(ctx, kv, P, start):
