@@ -679,14 +679,30 @@ int read_argmax(cw_model *m, uint32_t *out) {
     return CW_OK;
 }
 
-// The batched prompt phase of the n tokens in prompt_dev: every position
-// through every layer, kPrefillChunk at a time (the buffers hold one chunk),
+// Positions of one pass of the batched prompt phase (its buffers hold them).
+constexpr int kPrefillChunk = 4096;
+
+// Whether a prompt of n tokens goes through run_prefill, its buffers then being
+// there: head_dim 128 (what its attention is built for) and more than one
+// position (two 8B layers: 118 us for one token by a step, 205 for two, 293 for
+// three; 192 for a batch of 2 to 8; four 0.6B layers: 133, 249 and 358 against
+// 210).  With no room for the buffers it goes step by step.
+int plan_prompt(cw_model *m, int n, bool *batched) {
+    *batched = false;
+    if (m->cfg.head_dim != 128 || n < 2) return CW_OK;
+    const int rc = ensure_prefill(m, std::min(n, kPrefillChunk));
+    *batched = rc == CW_OK;
+    if (rc != CW_ERR_OOM) return rc;
+    (void)hipGetLastError();
+    return CW_OK;
+}
+
+// The batched prompt phase of the n tokens in prompt_dev (plan_prompt said it
+// runs): every position through every layer, kPrefillChunk at a time,
 // then the last position's logits and argmax, advancing the decode state when
 // given.  *last: its hidden row.
-constexpr int kPrefillChunk = 4096;
 int run_prefill(cw_model *m, int n, int start, GenState *state, const float **last) {
     const auto &c = m->cfg;
-    CW_TRY(ensure_prefill(m, std::min(n, kPrefillChunk)));
     int rows = 0;
     for (int i = 0; i < n; i += rows) {
         rows = std::min(n - i, kPrefillChunk);
@@ -705,12 +721,6 @@ int run_prefill(cw_model *m, int n, int start, GenState *state, const float **la
     return launch_lm_head_argmax(m->ctx, g, m->lm_scratch, m->argmax_out, state, m->prompt_dev,
                                  m->tokens_dev);
 }
-
-// Prompts that go through run_prefill: head_dim 128 (what its attention is
-// built for) and more than one position (two 8B layers: 118 us for one token
-// by a step, 205 for two, 293 for three; 192 for a batch of 2 to 8; four 0.6B
-// layers: 133, 249 and 358 against 210).
-bool batched_prompt(const cw_model *m, int n) { return m->cfg.head_dim == 128 && n > 1; }
 
 int require_final(cw_model *m, const char *what) {
     if (!m->finalized) {
@@ -1227,16 +1237,11 @@ int cw_generate(cw_model *m, const uint32_t *prompt, int n_prompt, int max_new, 
                      prompt[i]);
     CW_TRY(stage_prompt(m, prompt, n_prompt));
     int steps = (int)total;
-    bool batched = mode == CW_STEP_GRAPH && batched_prompt(m, n_prompt);
+    bool batched = false;
+    if (mode == CW_STEP_GRAPH) CW_TRY(plan_prompt(m, n_prompt, &batched));
     if (batched) {
         // the prompt's forwards at once; the LM head then advances the state
         // as the last of them would
-        const int rc = ensure_prefill(m, std::min(n_prompt, kPrefillChunk));
-        batched = rc == CW_OK;
-        if (rc != CW_OK && rc != CW_ERR_OOM) return rc;
-        if (!batched) (void)hipGetLastError();  // no room for its buffers: step by step
-    }
-    if (batched) {
         const int at = start_pos + n_prompt - 1;
         CW_TRY(set_state(m, GenState{at, prompt[n_prompt - 1], start_pos, n_prompt, 0, max_new}));
         const float *last = nullptr;
@@ -1268,7 +1273,9 @@ int cw_model_prefill(cw_model *m, const uint32_t *tokens, int n, int start_pos,
                      tokens[i]);
     CW_TRY(stage_prompt(m, tokens, n));
     const float *last = nullptr;
-    if (batched_prompt(m, n)) {
+    bool batched = false;
+    CW_TRY(plan_prompt(m, n, &batched));
+    if (batched) {
         CW_TRY(run_prefill(m, n, start_pos, nullptr, &last));
     } else {
         CW_TRY(set_state(m, GenState{start_pos, tokens[0], start_pos, n, 0, 0}));

@@ -267,7 +267,8 @@ int cw_model_tap(cw_model *m, const char *name, int layer, float *host_out, int 
  * max_new produced tokens (P+N-1 forwards), the whole step device-resident
  * (position and token live on the device), executed as `mode` (CW_STEP_*).
  * In CW_STEP_GRAPH mode with head_dim 128 a prompt of two or more tokens runs
- * as one batch (as in cw_model_prefill) and the replayed steps follow.
+ * as one batch (as in cw_model_prefill, where there is room for its buffers)
+ * and the replayed steps follow.
  * The first prompt token is fed at start_pos (0 = empty cache).  Writes
  * max_new ids to out_tokens.  CW_STEP_FUSED returns CW_ERR_ARG for shapes it
  * does not cover and CW_ERR_HIP if a grid barrier timed out. */
@@ -319,7 +320,8 @@ int cw_step_dry_plan(const cw_model_config *cfg, int n_cu, int split_gate_up, vo
  * the logits of all but the last discarded) for n tokens at positions
  * start_pos..start_pos+n-1, batched: each layer runs as Q4_0 GEMMs on the
  * matrix cores and causal attention over the cache (head_dim 128 and n > 1;
- * otherwise the per-token step runs n times).  Writes the KV
+ * otherwise, and where device memory has no room for the batch's buffers, the
+ * per-token step runs n times).  Writes the KV
  * rows, leaves the last position's logits (cw_model_logits) and final-normed
  * hidden state (cw_model_hidden), returns its argmax in *next_token, and sets
  * the decode state to (next_token, start_pos + n). */
