@@ -59,8 +59,9 @@ GEMM_EDGES = [(m, k, n) for m in (1, 15, 17, 33, 63, 65, 129)
 def test_q4_gemm_tile_edges(ctx, m, in_f, out_f):
     """Every element against an f64 product of the exactly dequantized
     weights.  The operands are exact to 2^-23 and the sums are f32: the same
-    bound as above, 2e-5 * sum_k |w x| (2^-24 per add over at most 1,280
-    blocks stays below it by a factor of 4)."""
+    bound as above, 2e-5 * sum_k |w x| (at most 15 + 80 + 15 additions of 2^-24
+    in a chain of 16 blocks, the chains of 1,280 blocks and 16 K splits, and two
+    more in a block's sum: 6.7e-6)."""
     s, q = cw.synth_q4(cw.synth_key(25, f"e{out_f}x{in_f}"), out_f, in_f, 0.02)
     x = cw.synth_normal_f32(cw.synth_key(25, f"ex{m}x{in_f}"), m * in_f).reshape(m, in_f)
     y = ctx.q4_gemm(ctx.storage(x), m, ctx.storage(s), ctx.storage(q), in_f, out_f).download()
@@ -68,6 +69,37 @@ def test_q4_gemm_tile_edges(ctx, m, in_f, out_f):
     x64 = x.astype(np.float64)
     err = np.abs(y.reshape(m, out_f) - x64 @ w.T)
     assert np.all(err <= 2e-5 * (np.abs(x64) @ np.abs(w).T) + 1e-30)
+
+
+# Rows of x in long segments, whose split keeps six chunks a thread (segments of
+# over 4,096 elements, four rows a workgroup) or reads the rest of a segment
+# above 12,288 elements again (by one row and by four); with the launches that
+# show how the plan splits K (not at all: the segment is the whole row)
+GEMM_LONG_ROWS = [(64, 65568, 70, "q4_gemm_splitk"), (1030, 12320, 70, "q4_gemm_splitk"),
+                  (900, 12800, 6144, "q4_gemm"), (1500, 12800, 4096, "q4_gemm")]
+
+
+@pytest.mark.parametrize("m,in_f,out_f,launch", GEMM_LONG_ROWS)
+def test_q4_gemm_long_rows(ctx, m, in_f, out_f, launch):
+    """Sampled rows and columns (the last of each among them) within
+    2e-5 * sum_k |w x| of 64 bits, as above."""
+    rng = np.random.default_rng(28)
+    s = np.abs(0.02 * rng.standard_normal((out_f, in_f // 32), np.float32)).astype(np.float16)
+    q = rng.integers(0, 256, (out_f, in_f // 32, 16), np.uint8)
+    x = rng.standard_normal((m, in_f), np.float32)
+    dev = [ctx.storage(v) for v in (x, s.view(np.uint16), q)]
+    ctx.profile_begin()
+    y = ctx.q4_gemm(dev[0], m, dev[1], dev[2], in_f, out_f).download().reshape(m, out_f)
+    labels = [r[0] for r in ctx.profile_report()]
+    for d in dev:
+        ctx.free(d)
+    assert launch in labels, labels
+    rows = np.unique(np.linspace(0, m - 1, 40).astype(int))
+    cols = np.unique(np.linspace(0, out_f - 1, 70).astype(int))
+    w = orc.dequant_q4_0_soa(s[cols].view(np.uint16), q[cols]).reshape(len(cols), in_f)
+    w, x = w.astype(np.float64), x[rows].astype(np.float64)
+    err = np.abs(y[np.ix_(rows, cols)] - x @ w.T)
+    assert np.all(err <= 2e-5 * (np.abs(x) @ np.abs(w).T))
 
 
 def test_q4_gemm_scales_at_odd_addresses(ctx):
@@ -276,6 +308,53 @@ def test_prefill_after_a_longer_one(ctx):
         logits.append(m.logits())
         m.close()
     assert float(np.max(np.abs(logits[0] - logits[1]))) <= 1e-4
+
+
+@pytest.mark.parametrize("P,launch", [(3, "q4_gemm_reduce_split"), (40, "prefill_split_rmsnorm")])
+def test_prefill_rows_above_12288(ctx, P, launch):
+    """A hidden state wider than the 12,288 elements that the split passes keep
+    in registers: the embedding pass, the sum of partials (few rows) and the
+    plain normalised split (more rows) read or store the rest of a row twice.
+    Logits within 1e-3 of the oracle's."""
+    cfg = cw.make_config(1, 12832, 4, 2, 128, 1024, 300, 48, cw.CW_F32, 1e-6, 1e6)
+    weights = cw.synthetic_weights(cfg, 88)
+    prompt = cw.synth_tokens(cw.synth_key(88, f"p{P}"), P, cfg.vocab)
+    m = cw.Model(ctx, cfg)
+    m.set_weights(weights)
+    m.finalize()
+    ctx.profile_begin()
+    nxt = m.prefill(prompt)
+    labels = [r[0] for r in ctx.profile_report()]
+    assert launch in labels, labels
+    o = orc.OracleModel(cfg, weights)
+    ref = oracle_prompt_logits(o, prompt)
+    o.close()
+    diff = float(np.max(np.abs(m.logits() - ref)))
+    assert diff <= LOGIT_TOL, diff
+    assert nxt == int(np.argmax(ref))
+    m.close()
+
+
+@pytest.mark.parametrize("kv,tol", [(cw.CW_F16, LOGIT_TOL), (cw.CW_F32, 2e-5)])
+@pytest.mark.parametrize("P", [4097, 4133])
+def test_prefill_beyond_one_chunk(ctx, kv, tol, P):
+    """A prompt longer than the 4,096 positions of one pass (the rest one row,
+    and several): the logits of the same prompt in two calls of fewer (f32 sums
+    in another order; with an f16 cache also ties), and generate's first id."""
+    cfg = cw.make_config(1, 256, 4, 2, 128, 512, 500, 4200, kv, 1e-6, 1e6)
+    weights = cw.synthetic_weights(cfg, 89)
+    prompt = cw.synth_tokens(cw.synth_key(89, f"p{P}"), P, cfg.vocab)
+    m = cw.Model(ctx, cfg)
+    m.set_weights(weights)
+    m.finalize()
+    nxt = m.prefill(prompt)
+    logits = m.logits()
+    assert m.generate(prompt, 2)[0] == nxt
+    m.prefill(prompt[:2000])
+    assert m.prefill(prompt[2000:], start_pos=2000) == nxt
+    diff = float(np.max(np.abs(m.logits() - logits)))
+    m.close()
+    assert diff <= tol, diff
 
 
 @pytest.mark.parametrize("n_heads,n_kv", [(4, 4), (8, 1), (16, 2)])
@@ -507,9 +586,9 @@ def test_prefill_rows_past_the_prompt_do_not_reach_it(ctx):
         assert np.array_equal(out[0], out[1])
 
 
-def test_prefill_f32_cache_runs_per_token(ctx):
-    """An f32 cache takes the per-token step for the prompt: same logits as
-    the oracle's loop."""
+def test_prefill_other_head_sizes_run_per_token(ctx):
+    """Head sizes other than 128 (here 16, with an f32 cache) take the per-token
+    step for the prompt: same logits as the oracle's loop."""
     cfg = cw.make_config(2, 64, 4, 2, 16, 128, 256, 20, cw.CW_F32, 1e-6, 1e6)
     weights = cw.synthetic_weights(cfg, 79)
     prompt = np.array([3, 1, 4, 1, 5, 9, 2, 6], np.uint32)
