@@ -306,8 +306,8 @@ struct GemmArgs {
 size_t gemm_img_elems(int M, int K);
 // Floats of its row scales (any number of segments).
 size_t gemm_rowscale_floats(int M);
-// padded scales of N rows of K, for matrices whose scales the GEMM cannot
-// read in pairs (0: not needed)
+// padded scales of N rows of K, for matrices whose scales the GEMM cannot read
+// in groups of eight blocks at 16-byte addresses (0: not needed)
 size_t gemm_spad_elems(int N, int K, const void *scales);
 // floats of split-K partials the GEMM's plan takes for this shape (0: none);
 // with less room it takes the best plan that fits
@@ -328,9 +328,9 @@ int launch_q4_gemm(cw_ctx *ctx, Epi epi, GemmArgs a, int *splits);
 // y = [resid +] the sum in order of a.part's `splits` partials
 int launch_gemm_reduce(cw_ctx *ctx, const GemmArgs &a, int splits);
 // The GEMM's result (its partials summed in the same pass) as the next GEMM's
-// split image, RMS-normalised with norm_w when set; y holds it too, but for
-// SwiGLU partials.  seg_blocks (SwiGLU partials only): row scales per that many
-// blocks, the K splits of the GEMM that follows.
+// split image, RMS-normalised with norm_w when set (EPI_ADD: always); y holds it
+// too, but for SwiGLU partials.  seg_blocks, without norm_w: row scales per that
+// many blocks, the K splits of the GEMM that follows.
 int launch_reduce_split(cw_ctx *ctx, Epi epi, const GemmArgs &a, int splits, const float *norm_w,
                         float eps, int seg_blocks, uint16_t *img, float *rowscale);
 // Blocks per K split of the GEMM's plan (as launch_q4_gemm will take it).

@@ -359,10 +359,10 @@ struct GT {
     static constexpr int BM = 16 * RT * WM, BN = 16 * CT * WN;
     static constexpr int WAVES = WM * WN, THREADS = 64 * WAVES;
     // one stage in LDS: x [row tile][block][hi | lo][lane] x 16 B, quants
-    // [column][slot] x 16 B; beside the stages, the scales of GROUPS groups
-    // of eight blocks, [column] x 16 B each (those of the stages in flight)
+    // [column][slot] x 16 B; beside the stages, the scales of two groups of
+    // eight blocks, [column] x 16 B each (those of the stages in flight)
     static constexpr int OQ = BM * SB * 128, BUF = OQ + BN * SB * 16;
-    static constexpr int GROUPS = NBUF * SB > 12 ? 4 : 2;
+    static constexpr int GROUPS = 2;
     static constexpr int OD = NBUF * BUF, LDS = OD + GROUPS * BN * 16;
     // 64-lane DMAs: of one stage by kind (a wave issues PX + PQ of them), and
     // of one group's scales (PD each by the first DW waves)
@@ -373,7 +373,7 @@ struct GT {
                   "every wave issues whole DMAs");
     static_assert(8 % SB == 0 && kChain % 8 == 0, "groups and chains are whole stages");
     static_assert(BM <= 64 && WM == 1, "a lane holds a row's scale");
-    static_assert(NBUF <= 3 || (NBUF - 2) * SB == 8, "one new group among the stages in flight");
+    static_assert(NBUF <= 3 && NBUF * SB <= 12, "one new group among the stages in flight");
     static_assert(LDS <= 160 * 1024, "LDS");
     static_assert((NBUF - 1) * PENDING + PD < 64, "wait count");
 };
@@ -625,9 +625,6 @@ void q4_gemm_kernel(cwi::GemmArgs a, int MT, int NT, int S, int per) {
         constexpr int AHEAD = G::NBUF - 2;
         if (AHEAD == 0 || st + AHEAD >= n_st) {
             wait_vm<0>();
-        } else if (AHEAD * SB % 8 == 0) {  // whole groups
-            if (wave < G::DW) wait_vm<AHEAD * G::PENDING + AHEAD * SB / 8 * G::PD>();
-            else wait_vm<AHEAD * G::PENDING>();
         } else if ((kb0 + (st + 1) * SB) % 8 == 0 && wave < G::DW) {
             wait_vm<AHEAD * G::PENDING + G::PD>();
         } else {
@@ -768,6 +765,11 @@ void q4_gemm_kernel(cwi::GemmArgs a, int MT, int NT, int S, int per) {
 // fit of a tile of less than 64 rows holds for one or two row tiles, which is
 // all it is used for: more of them read W again for too few rows (512 rows of
 // 4096 -> 6144 as 32 x 128 tiles: 83.7 us, as 64 x 128 in two splits 67.9).
+// Each of those launches was repeated on the same W, which the 256 MB
+// last-level cache then holds: mb is that cache's rate, not HBM's.  First calls
+// on new operands take longer at every size (16 rows of 4096 -> 12288: 29 us
+// with the passes around it, 16.5 repeated), and their plans may not be the
+// best there.
 struct Tile {
     int bm, bn, occ;
     float launch, round, share, mb, part;
@@ -853,10 +855,15 @@ int launch_split_image(cw_ctx *ctx, const char *label, SplitArgs a, int rows, in
     const int nt = std::min(512, (a.seg + 63) / 64 * 64);
     const int segs = (a.K / 8 + a.seg - 1) / a.seg;
     a.M = rows;
-    // four rows a workgroup where that still gives every CU one, for plain rows;
-    // counted with a row's segments only above 256 chunks each (512 rows of 12288
-    // in four: 9.9 us, 13.4 by single rows; of 4096 in two: 7.1 against 6.1)
-    // (merging the attention chunks of 512 rows so took 16 us, 8.4 by single rows)
+    // four rows a workgroup where that still gives every CU one, for plain rows
+    // with long segments.  Timed both ways for 64 to 3000 rows of 1024 to 16384
+    // in the segments of their plans: with 384 chunks and more a segment four
+    // rows take 0.66-1.03 of the time of single rows (512 rows of 12288 in four
+    // segments 9.5 against 13.0 us, 3000 in one 60 against 74), with 256 and a
+    // whole row 0.86-1.04, with 256 and several segments 0.80-1.08 (with 1,024
+    // rows 0.86-0.98), with 192 and fewer 1.0-2.1 once the chip is full (512
+    // rows of 4096 in eight of 64: 12.4 against 7.9).  (Merging the attention
+    // chunks of 512 rows so took 16 us, 8.4 by single rows.)
     if constexpr (SRC == SRC_ROWS) {
         if ((rows >= 4 * ctx->n_cu && a.seg >= 256) ||
             (rows * segs >= 4 * ctx->n_cu && a.seg > 256)) {
@@ -998,8 +1005,7 @@ int launch_reduce_split(cw_ctx *ctx, Epi epi, const GemmArgs &g, int splits, con
     if (epi == EPI_SWIGLU)
         return launch_split_image<false, SRC_SWIGLU>(ctx, "q4_gemm_reduce_swiglu", a, g.M,
                                                      seg_blocks);
-    return norm_w ? launch_split_image<true, SRC_PART>(ctx, "q4_gemm_reduce_split", a, g.M)
-                  : launch_split_image<false, SRC_PART>(ctx, "q4_gemm_reduce_split", a, g.M);
+    return launch_split_image<true, SRC_PART>(ctx, "q4_gemm_reduce_split", a, g.M);
 }
 
 }  // namespace cwi
