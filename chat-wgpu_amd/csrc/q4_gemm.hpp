@@ -491,14 +491,14 @@ __device__ __forceinline__ int w_row(int c, bool *up) {
 // 3000-token prompts 1-2 %).
 //
 // Bound, at 512 rows, by the chain of dequantization, MFMAs and scale FMAs,
-// which the operands' DMAs overlap only in part (matrix cores busy 30-44 %; 4096
+// which the operands' DMAs overlap only in part (matrix cores busy 29-42 %; 4096
 // -> 6144 with row-major x: 73.7 us, 53 without DMA, 90 with DMA alone); at few
 // rows by the launch, the first loads and W at about 2.3 TB/s.  Four waves side
 // by side along N dequantize every weight once; tiles of 16 and 32 rows keep
 // few rows from paying for padding.  128 x 128 tiles with row-major x took, with the passes around them,
 // 43.1 us for 16 rows of 4096 -> 12288 (here 16.5, this kernel 40.3 -> 11.5),
 // 52.2 for 100 of 12288 -> 4096 (here 41.5), 86.5 for 512 of 4096 -> 6144 (here
-// 69.6).
+// 70.5).
 template <int EPI, int OUT, class G, int OCC>
 __global__ __launch_bounds__(G::THREADS) __attribute__((amdgpu_waves_per_eu(OCC, OCC)))
 void q4_gemm_kernel(cwi::GemmArgs a, int MT, int NT, int S, int per) {
@@ -761,7 +761,8 @@ void q4_gemm_kernel(cwi::GemmArgs a, int MT, int NT, int S, int per) {
 // part * partials, where a workgroup runs `blocks` K blocks, load is the
 // workgroups of the busiest CU, rounds is load over the occ workgroups that
 // a CU holds, and W and the partials are in MB.  The plan with the least cost
-// is within 1.3 % of the best of the timed ones on average (23 % at most).  The
+// is within 1.3 % of the best of the timed ones on average (23 % at most; timed
+// before sums went in chains, which cost 64-row tiles up to 2 %).  The
 // fit of a tile of less than 64 rows holds for one or two row tiles, which is
 // all it is used for: more of them read W again for too few rows (512 rows of
 // 4096 -> 6144 as 32 x 128 tiles: 83.7 us, as 64 x 128 in two splits 67.9).
