@@ -293,7 +293,7 @@ struct GemmArgs {
     const uint16_t *sB;
     const uint8_t *qB;
     int s_stride;               // set by launch_q4_gemm: blocks per row of sA / sB
-    uint16_t *s_pad;            // room for padded scales (gemm_spad_elems), else null
+    uint16_t *s_pad;            // padded scales (gemm_scale_pad), where they are needed
     const float *resid;  // EPI_ADD: [M][N]
     float *y;            // [M][N]
     int M, N, K;
@@ -312,15 +312,26 @@ size_t gemm_spad_elems(int N, int K, const void *scales);
 // floats of split-K partials the GEMM's plan takes for this shape (0: none);
 // with less room it takes the best plan that fits
 size_t gemm_part_floats(const cw_ctx *ctx, Epi epi, int M, int N, int K);
+// The copy of a GEMM's scales to padded rows, made by the pass that makes its x
+// image (mats 0: it reads them as they are): of one matrix, or SwiGLU's two, of N
+// rows of nb blocks, into dst (gemm_spad_elems of each, GemmArgs::s_pad).
+struct ScalePad {
+    int mats, N, nb;
+    const uint16_t *src[2];
+    uint16_t *dst;
+};
+ScalePad gemm_scale_pad(Epi epi, const uint16_t *sA, const uint16_t *sB, int N, int K,
+                        uint16_t *dst);
 // The split image of rows of x, RMS-normalised with norm_w when set; without,
-// a row scale per seg_blocks blocks (0: per row).
+// a row scale per seg_blocks blocks (0: per row).  pad, here and below: the
+// scales of the GEMM that follows.
 int launch_split_rows(cw_ctx *ctx, const float *x, const float *norm_w, float eps, int rows, int K,
-                      uint16_t *img, float *rowscale, int seg_blocks);
+                      uint16_t *img, float *rowscale, int seg_blocks, const ScalePad &pad);
 // The embedding rows of `rows` tokens (ids on the device, validated < vocab by
 // the caller) into y, and their RMS-normalised split image.
 int launch_embed_split(cw_ctx *ctx, const float *table, const uint32_t *tok_dev,
                        const float *norm_w, float eps, int rows, int K, float *y, uint16_t *img,
-                       float *rowscale);
+                       float *rowscale, const ScalePad &pad);
 // *splits = 0 when y was written, else the K splits whose partials are in
 // a.part (a.resid not yet added): [split][M][N], for SwiGLU [split][gate |
 // up][M][N].
@@ -332,7 +343,8 @@ int launch_gemm_reduce(cw_ctx *ctx, const GemmArgs &a, int splits);
 // too, but for SwiGLU partials.  seg_blocks, without norm_w: row scales per that
 // many blocks, the K splits of the GEMM that follows.
 int launch_reduce_split(cw_ctx *ctx, Epi epi, const GemmArgs &a, int splits, const float *norm_w,
-                        float eps, int seg_blocks, uint16_t *img, float *rowscale);
+                        float eps, int seg_blocks, uint16_t *img, float *rowscale,
+                        const ScalePad &pad);
 // Blocks per K split of the GEMM's plan (as launch_q4_gemm will take it).
 int gemm_seg_blocks(const cw_ctx *ctx, Epi epi, int M, int N, int K, size_t part_floats);
 constexpr int kMaxSplits = 16;  // row scale sets at most
@@ -367,7 +379,7 @@ int launch_attn_prefill(cw_ctx *ctx, const AttnPrefillPlan &p, AttnPrefillArgs a
 // The rows' split image for the O projection: of a.out, or of the merged chunks
 // (row scales per seg_blocks blocks).
 int launch_attn_split(cw_ctx *ctx, const AttnPrefillPlan &p, const AttnPrefillArgs &a,
-                      int seg_blocks, uint16_t *img, float *rowscale);
+                      int seg_blocks, uint16_t *img, float *rowscale, const ScalePad &pad);
 
 // ---- the fused decode step (one persistent cooperative kernel per token)
 

@@ -598,9 +598,14 @@ int enqueue_prefill(cw_model *m, int tok, int n, int start) {
     const auto &c = m->cfg;
     const float eps = c.eps;
     // a GEMM's result as the next one's operand, in one pass
-    auto to_image = [&](Epi epi, const GemmArgs &a, int splits, const float *norm_w, int seg) {
+    auto to_image = [&](Epi epi, const GemmArgs &a, int splits, const float *norm_w, int seg,
+                        const ScalePad &pad) {
         return launch_reduce_split(ctx, epi, a, splits, norm_w, eps, seg, m->pf_img,
-                                   m->pf_rowscale);
+                                   m->pf_rowscale, pad);
+    };
+    // the scales of the GEMM that follows a pass
+    auto pad_of = [&](const Q4W &w) {
+        return gemm_scale_pad(EPI_STORE, w.s, nullptr, w.out_f, w.in_f, m->pf_spad);
     };
     // the K splits of the O and down GEMMs, for their operands' row scales
     const int seg_o = gemm_seg_blocks(ctx, EPI_ADD, n, c.dim, m->q_dim, m->pf_part_floats);
@@ -608,7 +613,8 @@ int enqueue_prefill(cw_model *m, int tok, int n, int start) {
     GemmArgs g{};
     int splits = 0;
     CW_TRY(launch_embed_split(ctx, m->embed, m->prompt_dev + tok, m->layers[0].attn_norm, eps, n, c.dim,
-                              m->pf_hidden, m->pf_img, m->pf_rowscale));
+                              m->pf_hidden, m->pf_img, m->pf_rowscale,
+                              pad_of(m->layers[0].qkv)));
     const AttnPrefillPlan plan = attn_prefill_plan(ctx, c.kv_dtype, n, c.n_heads, c.n_kv_heads,
                                                    start, m->pf_attn_rows);
     AttnPrefillArgs at{};
@@ -635,17 +641,20 @@ int enqueue_prefill(cw_model *m, int tok, int n, int start) {
         at.kc = kc;
         at.vc = vc;
         CW_TRY(launch_attn_prefill(ctx, plan, at, c.kv_dtype));
-        CW_TRY(launch_attn_split(ctx, plan, at, seg_o, m->pf_img, m->pf_rowscale));
+        CW_TRY(launch_attn_split(ctx, plan, at, seg_o, m->pf_img, m->pf_rowscale, pad_of(L.wo)));
         CW_TRY(pf_gemm(m, n, m->q_dim, EPI_ADD, L.wo, nullptr, m->pf_hidden, m->pf_hidden, &g,
                        &splits, seg_o));
-        CW_TRY(to_image(EPI_ADD, g, splits, L.ffn_norm, 0));
+        CW_TRY(to_image(EPI_ADD, g, splits, L.ffn_norm, 0,
+                        gemm_scale_pad(EPI_SWIGLU, L.gate.s, L.up.s, c.hidden, c.dim,
+                                       m->pf_spad)));
         CW_TRY(tap_row(m, m->tap_post + (size_t)i * c.dim, m->pf_hidden, n - 1, c.dim));
         CW_TRY(pf_gemm(m, n, c.dim, EPI_SWIGLU, L.gate, &L.up, nullptr, m->pf_act, &g, &splits));
-        CW_TRY(to_image(EPI_SWIGLU, g, splits, nullptr, seg_d));
+        CW_TRY(to_image(EPI_SWIGLU, g, splits, nullptr, seg_d, pad_of(L.down)));
         CW_TRY(pf_gemm(m, n, c.hidden, EPI_ADD, L.down, nullptr, m->pf_hidden, m->pf_hidden, &g,
                        &splits, seg_d));
         if (i + 1 < c.n_layers)
-            CW_TRY(to_image(EPI_ADD, g, splits, m->layers[i + 1].attn_norm, 0));
+            CW_TRY(to_image(EPI_ADD, g, splits, m->layers[i + 1].attn_norm, 0,
+                            pad_of(m->layers[i + 1].qkv)));
         else if (splits)
             CW_TRY(launch_gemm_reduce(ctx, g, splits));
         CW_TRY(tap_row(m, m->tap_out + (size_t)i * c.dim, m->pf_hidden, n - 1, c.dim));

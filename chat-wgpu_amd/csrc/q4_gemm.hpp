@@ -84,9 +84,10 @@ struct SplitArgs {
     const float *norm_w;  // NORM: gain [K]
     float eps;
     int K;
-    int seg;  // chunks per segment
+    int seg, segs;  // chunks per segment, segments
     uint16_t *img;
     float *rowscale;
+    cwi::ScalePad pad;  // copied by the workgroups past the segments
 };
 
 __device__ __forceinline__ float2 add(float2 a, float2 b) {
@@ -125,12 +126,38 @@ __device__ __forceinline__ float4 sum4(const float *p, int S, size_t stride) {
 
 __device__ __forceinline__ float silu_mul(float g, float u) { return g / (1.0f + expf(-g)) * u; }
 
+// Scales whose rows are not whole groups of eight blocks (or whose address is
+// not a multiple of 16), copied to rows that are: the GEMM loads them a group
+// (16 bytes) at a time.  A part of the pass that makes the x image, as
+// workgroups of their own (a launch of its own before: 4 rows of 288 -> 512 14.0
+// us in all, 8.8-10.4 so).
+__device__ __forceinline__ void copy_scales(const cwi::ScalePad &p, size_t at, size_t step) {
+    const int ns = (p.nb + 7) / 8 * 8;
+    const size_t total = (size_t)p.N * ns;
+    for (int m = 0; m < p.mats; ++m)
+        for (size_t i = at; i < total; i += step) {
+            const size_t n = i / ns;
+            const int b = (int)(i - n * ns);
+            p.dst[m * total + i] = p.src[m][n * p.nb + min(b, p.nb - 1)];
+        }
+}
+
 // With R = 4 a workgroup takes four rows, neighbouring lanes the same chunk of
 // each, so a store covers 64 bytes of an image line instead of 16 (3000 rows of
 // 12288: 58 us; 80 with one row, 141 with one row and in plain row order).
-template <bool NORM, int SRC, int CH, int R>
+// PAD: the launch has workgroups that copy scales (a variant, since the test in
+// front of the loads costs the others 0.2 us).
+template <bool NORM, int SRC, int CH, int R, bool PAD>
 __global__ __launch_bounds__(R == 1 ? 512 : 1024) void split_image_kernel(SplitArgs a) {
     __shared__ float red[2][R == 1 ? 8 : 16][R];
+    if constexpr (PAD) {
+        if ((int)blockIdx.y >= a.segs) {
+            const size_t wg = (size_t)(blockIdx.y - a.segs) * gridDim.x + blockIdx.x;
+            copy_scales(a.pad, wg * blockDim.x + threadIdx.x,
+                        (size_t)(gridDim.y - a.segs) * gridDim.x * blockDim.x);
+            return;
+        }
+    }
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     // this thread's row of the workgroup's, and its place among that row's threads
     const int ri = threadIdx.x % R, tid = threadIdx.x / R, nt = blockDim.x / R;
@@ -330,20 +357,6 @@ __global__ __launch_bounds__(kT) void gemm_reduce_kernel(const float *__restrict
         float v = part[e];
         for (int s = 1; s < S; ++s) v += part[(size_t)s * n + e];
         y[e] = resid ? resid[e] + v : v;
-    }
-}
-
-// Scales whose rows are not whole groups of eight blocks (or whose address is
-// not a multiple of 16), copied to rows that are: the GEMM loads them a group
-// (16 bytes) at a time.
-__global__ __launch_bounds__(kT) void pad_scales_kernel(const uint16_t *__restrict__ s, int nb,
-                                                        int ns, size_t total,
-                                                        uint16_t *__restrict__ out) {
-    for (size_t i = (size_t)blockIdx.x * kT + threadIdx.x; i < total;
-         i += (size_t)gridDim.x * kT) {
-        const size_t n = i / ns;
-        const int b = (int)(i - n * ns);
-        out[i] = s[n * nb + min(b, nb - 1)];
     }
 }
 
@@ -856,6 +869,17 @@ int launch_split_image(cw_ctx *ctx, const char *label, SplitArgs a, int rows, in
     const int nt = std::min(512, (a.seg + 63) / 64 * 64);
     const int segs = (a.K / 8 + a.seg - 1) / a.seg;
     a.M = rows;
+    a.segs = segs;
+    // gx workgroups per segment, then those that copy scales (four of them a
+    // thread, 4,096 workgroups at most)
+    auto go = [&](auto plain, auto padded, int gx, int threads) {
+        if (a.pad.mats == 0)
+            return cwi::launch(ctx, label, plain, dim3(gx, segs), dim3(threads), 0, a);
+        const size_t total = (size_t)a.pad.N * ((a.pad.nb + 7) / 8 * 8);
+        const int wgs = (int)std::min<size_t>((total + 4 * threads - 1) / (4 * threads), 4096);
+        return cwi::launch(ctx, label, padded, dim3(gx, segs + (wgs + gx - 1) / gx), dim3(threads),
+                           0, a);
+    };
     // four rows a workgroup where that still gives every CU one, for plain rows
     // with long segments.  Timed both ways for 64 to 3000 rows of 1024 to 16384
     // in the segments of their plans: with 384 chunks and more a segment four
@@ -868,18 +892,18 @@ int launch_split_image(cw_ctx *ctx, const char *label, SplitArgs a, int rows, in
     if constexpr (SRC == SRC_ROWS) {
         if ((rows >= 4 * ctx->n_cu && a.seg >= 256) ||
             (rows * segs >= 4 * ctx->n_cu && a.seg > 256)) {
-            const dim3 grid((rows + 3) / 4, segs);
-            if (a.seg <= 512)
-                return cwi::launch(ctx, label, split_image_kernel<NORM, SRC, 2, 4>, grid,
-                                   dim3(1024), 0, a);
-            return cwi::launch(ctx, label, split_image_kernel<NORM, SRC, 6, 4>, grid, dim3(1024),
-                               0, a);
+            return a.seg <= 512 ? go(split_image_kernel<NORM, SRC, 2, 4, false>,
+                                     split_image_kernel<NORM, SRC, 2, 4, true>, (rows + 3) / 4,
+                                     1024)
+                                : go(split_image_kernel<NORM, SRC, 6, 4, false>,
+                                     split_image_kernel<NORM, SRC, 6, 4, true>, (rows + 3) / 4,
+                                     1024);
         }
     }
-    const dim3 grid(rows, segs);
-    if (a.seg <= nt)
-        return cwi::launch(ctx, label, split_image_kernel<NORM, SRC, 1, 1>, grid, dim3(nt), 0, a);
-    return cwi::launch(ctx, label, split_image_kernel<NORM, SRC, 3, 1>, grid, dim3(nt), 0, a);
+    return a.seg <= nt ? go(split_image_kernel<NORM, SRC, 1, 1, false>,
+                            split_image_kernel<NORM, SRC, 1, 1, true>, rows, nt)
+                       : go(split_image_kernel<NORM, SRC, 3, 1, false>,
+                            split_image_kernel<NORM, SRC, 3, 1, true>, rows, nt);
 }
 
 }  // namespace
@@ -905,9 +929,17 @@ int gemm_seg_blocks(const cw_ctx *ctx, Epi epi, int M, int N, int K, size_t part
     return gemm_plan(ctx, epi, M, N, K, part_floats).per;
 }
 
+ScalePad gemm_scale_pad(Epi epi, const uint16_t *sA, const uint16_t *sB, int N, int K,
+                        uint16_t *dst) {
+    const bool two = epi == EPI_SWIGLU;
+    if (scales_in_groups(K, sA) && (!two || scales_in_groups(K, sB))) return ScalePad{};
+    return ScalePad{two ? 2 : 1, N, K / 32, {sA, sB}, dst};
+}
+
 int launch_split_rows(cw_ctx *ctx, const float *x, const float *norm_w, float eps, int rows, int K,
-                      uint16_t *img, float *rowscale, int seg_blocks) {
+                      uint16_t *img, float *rowscale, int seg_blocks, const ScalePad &pad) {
     SplitArgs a{};
+    a.pad = pad;
     a.x = x;
     a.norm_w = norm_w;
     a.eps = eps;
@@ -920,8 +952,9 @@ int launch_split_rows(cw_ctx *ctx, const float *x, const float *norm_w, float ep
 
 int launch_embed_split(cw_ctx *ctx, const float *table, const uint32_t *tok_dev,
                        const float *norm_w, float eps, int rows, int K, float *y, uint16_t *img,
-                       float *rowscale) {
+                       float *rowscale, const ScalePad &pad) {
     SplitArgs a{};
+    a.pad = pad;
     a.x = table;
     a.tok = tok_dev;
     a.y = y;
@@ -934,11 +967,13 @@ int launch_embed_split(cw_ctx *ctx, const float *table, const uint32_t *tok_dev,
 }
 
 int launch_attn_split(cw_ctx *ctx, const AttnPrefillPlan &p, const AttnPrefillArgs &t,
-                      int seg_blocks, uint16_t *img, float *rowscale) {
+                      int seg_blocks, uint16_t *img, float *rowscale, const ScalePad &pad) {
     const int K = t.n_heads * 128;
     if (p.chunks == 1)
-        return launch_split_rows(ctx, t.out, nullptr, 0.0f, t.M, K, img, rowscale, seg_blocks);
+        return launch_split_rows(ctx, t.out, nullptr, 0.0f, t.M, K, img, rowscale, seg_blocks,
+                                 pad);
     SplitArgs a{};
+    a.pad = pad;
     a.x = t.part;
     a.MK = (size_t)t.M * K;
     a.ml = t.ml;
@@ -956,17 +991,10 @@ int launch_q4_gemm(cw_ctx *ctx, Epi epi, GemmArgs a, int *splits) {
     const GemmPlan p = gemm_plan(ctx, epi, a.M, a.N, a.K, a.part ? a.part_floats : 0);
     const int nb = a.K / 32;
     a.s_stride = nb;
-    if (!scales_in_groups(a.K, a.sA) || (epi == EPI_SWIGLU && !scales_in_groups(a.K, a.sB))) {
+    if (gemm_scale_pad(epi, a.sA, a.sB, a.N, a.K, a.s_pad).mats) {
         a.s_stride = (nb + 7) / 8 * 8;
-        const size_t total = (size_t)a.N * a.s_stride;
-        const uint16_t **mats[2] = {&a.sA, &a.sB};
-        for (int i = 0; i < (epi == EPI_SWIGLU ? 2 : 1); ++i) {
-            uint16_t *out = a.s_pad + i * total;
-            const unsigned blocks = (unsigned)std::min<size_t>((total + kT - 1) / kT, 4096);
-            CW_TRY(launch(ctx, "q4_gemm_pad_scales", pad_scales_kernel, dim3(blocks), dim3(kT), 0,
-                          *mats[i], nb, a.s_stride, total, out));
-            *mats[i] = out;
-        }
+        a.sA = a.s_pad;
+        a.sB = a.s_pad + (size_t)a.N * a.s_stride;
     }
     *splits = p.S > 1 ? p.S : 0;
     switch (epi) {
@@ -989,8 +1017,10 @@ int launch_gemm_reduce(cw_ctx *ctx, const GemmArgs &a, int splits) {
 }
 
 int launch_reduce_split(cw_ctx *ctx, Epi epi, const GemmArgs &g, int splits, const float *norm_w,
-                        float eps, int seg_blocks, uint16_t *img, float *rowscale) {
+                        float eps, int seg_blocks, uint16_t *img, float *rowscale,
+                        const ScalePad &pad) {
     SplitArgs a{};
+    a.pad = pad;
     a.x = splits ? g.part : g.y;
     a.S = splits;
     a.MK = (size_t)g.M * g.N;
@@ -1002,7 +1032,7 @@ int launch_reduce_split(cw_ctx *ctx, Epi epi, const GemmArgs &g, int splits, con
     a.img = img;
     a.rowscale = rowscale;
     if (!splits)
-        return launch_split_rows(ctx, g.y, norm_w, eps, g.M, g.N, img, rowscale, seg_blocks);
+        return launch_split_rows(ctx, g.y, norm_w, eps, g.M, g.N, img, rowscale, seg_blocks, pad);
     if (epi == EPI_SWIGLU)
         return launch_split_image<false, SRC_SWIGLU>(ctx, "q4_gemm_reduce_swiglu", a, g.M,
                                                      seg_blocks);
@@ -1034,12 +1064,13 @@ extern "C" int cw_q4_gemm(cw_ctx *ctx, const float *x, int m, const uint16_t *sc
     uint16_t *img = reinterpret_cast<uint16_t *>(base);
     float *rs = reinterpret_cast<float *>(base + rs_off);
     a.seg_blocks = part ? gemm_seg_blocks(ctx, EPI_STORE, m, out_f, in_f, part) : 0;
-    CW_TRY(launch_split_rows(ctx, x, nullptr, 0.0f, m, in_f, img, rs, a.seg_blocks));
+    a.s_pad = reinterpret_cast<uint16_t *>(base + sp_off);
+    CW_TRY(launch_split_rows(ctx, x, nullptr, 0.0f, m, in_f, img, rs, a.seg_blocks,
+                             gemm_scale_pad(EPI_STORE, scales, nullptr, out_f, in_f, a.s_pad)));
     a.img = img;
     a.rowscale = rs;
     a.sA = scales;
     a.qA = quants;
-    a.s_pad = reinterpret_cast<uint16_t *>(base + sp_off);
     a.y = y;
     a.M = m;
     a.N = out_f;

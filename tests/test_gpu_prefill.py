@@ -71,6 +71,28 @@ def test_q4_gemm_tile_edges(ctx, m, in_f, out_f):
     assert np.all(err <= 2e-5 * (np.abs(x64) @ np.abs(w).T) + 1e-30)
 
 
+@pytest.mark.parametrize("m,in_f,out_f", [(4, 288, 512), (1, 32, 33000), (1000, 288, 513),
+                                          (3, 1056, 40000), (1030, 2080, 300)])
+def test_q4_gemm_padded_scales_take_no_launch(ctx, m, in_f, out_f):
+    """Scale rows that are not whole groups of eight blocks are copied by the
+    pass that splits x, by its own workgroups, few or many beside the rows':
+    no launch more than aligned rows take, and results within
+    2e-5 * sum_k |w x| of 64 bits."""
+    s, q = cw.synth_q4(cw.synth_key(29, f"p{out_f}x{in_f}"), out_f, in_f, 0.02)
+    x = cw.synth_normal_f32(cw.synth_key(29, f"px{m}x{in_f}"), m * in_f).reshape(m, in_f)
+    dev = [ctx.storage(v) for v in (x, s, q)]
+    ctx.profile_begin()
+    y = ctx.q4_gemm(dev[0], m, dev[1], dev[2], in_f, out_f).download().reshape(m, out_f)
+    launches = {r[0]: r[1] for r in ctx.profile_report()}
+    assert launches in ({"prefill_split": 1, "q4_gemm": 1},
+                        {"prefill_split": 1, "q4_gemm_splitk": 1, "q4_gemm_reduce": 1}), launches
+    rows = np.unique(np.linspace(0, m - 1, 30).astype(int))
+    w = orc.dequant_q4_0_soa(s, q).reshape(out_f, in_f).astype(np.float64)
+    x64 = x[rows].astype(np.float64)
+    err = np.abs(y[rows] - x64 @ w.T)
+    assert np.all(err <= 2e-5 * (np.abs(x64) @ np.abs(w).T) + 1e-30)
+
+
 # Rows of x in long segments, whose split keeps six chunks a thread (segments of
 # over 4,096 elements, four rows a workgroup) or reads the rest of a segment
 # above 12,288 elements again (by one row and by four); with the launches that
