@@ -281,7 +281,7 @@ int launch_argmax(cw_ctx *ctx, const float *logits, int n, uint32_t *out_dev, vo
 
 // ---- batched prefill (M positions per launch)
 
-// y[M][N] = x[M][K] . W[N][K]^T with x given as its split image (q4_gemm.hpp)
+// y[M][N] = x[M][K] . W[N][K]^T with x given as its split image (q4_gemm.hip)
 // and W split GGUF Q4_0; EPI_SWIGLU reads a second matrix (B) and stores
 // silu(A x) * (B x).
 struct GemmArgs {

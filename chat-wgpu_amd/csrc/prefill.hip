@@ -4,15 +4,19 @@
 // (model::generate runs P forwards, src/model/mod.rs:57-125; each forward is
 // Qwen3::forward, src/model/qwen3.rs:139-191).  This file computes the same
 // forward for M positions at once, with the linear layers as Q4_0
-// dequant-GEMMs on the matrix cores (q4_gemm.hpp) and causal attention as MFMA
+// dequant-GEMMs on the matrix cores (q4_gemm.hip) and causal attention as MFMA
 // tiles.
 //
 // Attention must match the f32 per-token path, so q and the softmax weights go
 // through the matrix cores as two f16 or as f32 (details at the kernel).
 
-#include "q4_gemm.hpp"
+#include <cmath>
+
+#include "prompt_device.hpp"
 
 namespace {
+
+using namespace cwi;
 
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll
@@ -110,7 +114,7 @@ __global__ __launch_bounds__(kT) void qk_rope_kv_kernel(const float *__restrict_
 // Key chunks: a workgroup takes `ct` key tiles of its rows' range, so that few
 // rows against many keys, and the long rows of a causal prompt, still spread
 // over the chip.  With more than one chunk it leaves (max, sum, o) partials,
-// which the pass that reads the rows merges (q4_gemm.hpp).
+// which the pass that reads the rows merges (q4_gemm.hip).
 //
 // Bound by the softmax's vector work and waits beside short MFMA runs (512
 // positions: matrix cores busy 7 %, waves waiting 39 % of their time), so the
