@@ -694,8 +694,10 @@ constexpr int kPrefillChunk = 4096;
 // Whether a prompt of n tokens goes through run_prefill, its buffers then being
 // there: head_dim 128 (what its attention is built for) and more than one
 // position (two 8B layers: 118 us for one token by a step, 205 for two, 293 for
-// three; 192 for a batch of 2 to 8; four 0.6B layers: 133, 249 and 358 against
-// 210).  With no room for the buffers it goes step by step.
+// three; 192 for a batch of 2 to 8; four 0.6B layers: 133, 254 and 344 against
+// 220; 28 of them: 1164-1185 for two and 1710-1740 for three against 1160-1200,
+// and up to 1370 in a process's first calls, whose launches the host holds up).
+// With no room for the buffers it goes step by step.
 int plan_prompt(cw_model *m, int n, bool *batched) {
     *batched = false;
     if (m->cfg.head_dim != 128 || n < 2) return CW_OK;
